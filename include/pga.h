@@ -444,15 +444,15 @@ PGA_API pga_status pga_lbvh_bounds(pga_lbvh* bvh, const float* aabbs, uint32_t n
 PGA_API pga_status pga_lbvh_build(pga_lbvh* bvh, const float* aabbs, uint32_t n, const float scene_min[3],
                                   const float scene_max[3], uint64_t* keys, int32_t* left, int32_t* right,
                                   int32_t* parent, int32_t* leaf_parent, float* node_aabb);
-/* device time of the last build (Morton codes to refit) */
+/* device time of the last build (Morton codes to tree) */
 PGA_API pga_status pga_lbvh_seconds(pga_lbvh* bvh, double* seconds);
 
 /* The build of pga_lbvh_build with no builder and no allocation. No
  * counterpart in the reference: it is for callers that cannot allocate
  * device memory (code recording a HIP graph, serving loops, harnesses that
- * forbid hipMalloc). The sort and refit scratch is a device array inside the
+ * forbid hipMalloc). The sort and tree scratch is a device array inside the
  * library, one per GPU, looked up with hipGetSymbolAddress on the first call
- * on that GPU and held until the process ends (about 24.3 MiB): at most
+ * on that GPU and held until the process ends (about 16.1 MiB): at most
  * PGA_LBVH_NOALLOC_MAX_LEAVES leaves, larger n is refused with
  * PGA_ERR_INVALID_ARG (message: pga_lbvh_last_error(NULL)). The build is
  * enqueued on `stream` (a hipStream_t of the current device; NULL: the

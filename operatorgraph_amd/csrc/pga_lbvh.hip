@@ -1,31 +1,29 @@
 // pga_lbvh.hip - linear BVH over terminal AABBs on gfx950 (wave64).
 //
-// The construction of GPUBVHConstructor.cuh (Karras 2012) in six steps:
+// The construction of GPUBVHConstructor.cuh (Karras 2012) in three steps:
 //   1. k_morton  - AABB centre normalised to the scene box, 10 bits per axis
 //                  interleaved into a 30-bit Morton code (GPUBVHConstructor.cuh:
-//                  44-86); the payload is the AABB index;
-//   2. LSD radix sort of (code, index) pairs, four 8-bit passes, each
-//                  k_hist -> scan (k_scan_reduce, k_scan_top, k_scan_down) ->
-//                  k_scatter; the scatter is stable (per-wave ranks from eight
-//                  ballots, per-workgroup digit cursors in LDS), so sorting the
-//                  codes of indices in ascending order gives the order of the
-//                  reference's unique 64-bit keys (code << 32 | index), which
-//                  thrust::sort orders (:311-312); the last pass writes those
-//                  keys directly;
-//   3. k_karras  - one thread per internal node: direction, range and split
-//                  by binary search over the common-prefix length of the
-//                  64-bit keys (buildRadixTree, :88-213); it also records the
-//                  far end of each node's leaf range;
-//   4. refit     - climbs from the leaves: the first child to reach a node
-//                  stops, the second unites both boxes and goes on
-//                  (propagateBVH's ticket, :215-261). k_refit_local completes
-//                  the nodes whose leaf range lies inside one workgroup's tile
-//                  of sorted leaves, through LDS; k_refit_global the nodes
-//                  spanning tiles, through global memory, where boxes are
-//                  written and read with agent-scope atomic loads and stores,
-//                  coherent across the XCDs' L2 caches without a full
-//                  write-back, and each store completes before the ticket of
-//                  the parent is taken.
+//                  44-86), written as the reference's unique 64-bit key
+//                  (code << 32 | index), with the digit histograms of all four
+//                  sort passes;
+//   2. LSD radix sort of the keys' codes, four 8-bit passes (thrust::sort,
+//                  :311-312, orders the same keys): k_digit_totals, then one
+//                  k_sweep per pass, which ranks a tile, finds the tile's place
+//                  by looking back over the tiles before it, and scatters it.
+//                  A stable sort of the codes of ascending indices gives the
+//                  order of the keys. Up to kSmallLeaves leaves one workgroup
+//                  sorts in LDS (k_sort_small);
+//   3. the tree  - the radix tree (buildRadixTree, :88-213) and its boxes
+//                  (propagateBVH, :215-261) in one climb from the leaves
+//                  (after Apetrei 2014): a subtree over the sorted leaves
+//                  [l, r] continues on the side of the closer neighbour, the
+//                  first child to reach a split leaves its end and box there,
+//                  the second unites both and goes on. k_tree_leaves climbs
+//                  inside a workgroup's tile of leaves, k_tree_roots inside a
+//                  group of the subtrees the previous level could not finish,
+//                  until one group is left; every exchange goes through LDS.
+//                  The numbering is the reference's: a right child [l, r] is
+//                  node l, a left child node r, the root node 0.
 // Children are encoded as in the reference: >= 0 a leaf (sorted position),
 // < 0 an internal node (negated index); node 0 is the root.
 //
@@ -45,12 +43,20 @@
 
 namespace bvhk {
 
-constexpr uint32_t kThreads = 256;
-constexpr uint32_t kItems = 16;
+constexpr uint32_t kThreads = 1024;              // sort and tree workgroups
+constexpr uint32_t kWaves = kThreads / 64u;
+constexpr uint32_t kItems = 4;
 constexpr uint32_t kTile = kThreads * kItems;   // keys per sort workgroup
-constexpr uint32_t kScanTile = 4096;            // histogram entries per scan workgroup
+constexpr uint32_t kSmallLeaves = kTile;        // up to here one workgroup sorts all keys in LDS
+constexpr uint32_t kDigits = 256, kPasses = 4;  // 30-bit codes: digits at bits 32, 40, 48, 56 of the key
+constexpr uint32_t kHistBlocks = 512;           // most workgroups of k_morton
 constexpr uint32_t kGatherBlocks = 8192;         // grid-stride workgroups of the terminal gather
-constexpr uint32_t kRefitTile = 1024;            // sorted leaves per refit workgroup (256 threads)
+constexpr uint32_t kTreeTile = 1024;             // sorted leaves per workgroup of the tree's first level
+constexpr uint32_t kTreeGroup = 32;              // workgroups of one level whose open subtrees one of the next takes
+constexpr uint32_t kMaxRoots = 128;              // open subtrees a workgroup may leave (see k_tree_leaves)
+typedef unsigned long long u64;
+// two floats of a box record: boxes are 24-byte records that a caller may align to 4 bytes only
+typedef float box2 __attribute__((ext_vector_type(2), aligned(4)));
 
 // leaf count: the host bound, or the device word when there is one
 __device__ __forceinline__ uint32_t leaf_count(uint32_t n, const uint32_t* nd) {
@@ -179,47 +185,106 @@ __global__ void __launch_bounds__(256) k_bounds_fold(float* part, uint32_t npart
     if (threadIdx.x < 6) part[threadIdx.x] = red[threadIdx.x][0];
 }
 
-// scene box from the host (mn, ex) or, with `box`, from the device: min xyz,
-// max xyz, an empty extent taken as 1
-__global__ void __launch_bounds__(256) k_morton(const float* __restrict__ aabbs, uint32_t n, const uint32_t* nd,
-                                                float mn0, float mn1, float mn2, float ex0, float ex1, float ex2,
-                                                const float* __restrict__ box,
-                                                uint32_t* __restrict__ code, uint32_t* __restrict__ idx) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= leaf_count(n, nd)) return;
-    if (box) {
-        mn0 = box[0]; mn1 = box[1]; mn2 = box[2];
-        ex0 = box[3] - mn0; ex1 = box[4] - mn1; ex2 = box[5] - mn2;
-        ex0 = ex0 > 0.0f ? ex0 : 1.0f; ex1 = ex1 > 0.0f ? ex1 : 1.0f; ex2 = ex2 > 0.0f ? ex2 : 1.0f;
+// Adds one to h[d] for every lane of `valid`: sorted or clustered input gives
+// whole waves one digit, which then costs one LDS atomic instead of 64 on the
+// same address.
+__device__ __forceinline__ void hist_add(uint32_t* h, uint32_t d, bool valid) {
+    const u64 m = __ballot(valid);
+    if (m == 0ull) return;
+    const int lead = __ffsll((long long)m) - 1;
+    const uint32_t d0 = __shfl(d, lead);
+    if (__ballot(valid && d != d0) == 0ull) {
+        if ((int)(threadIdx.x & 63u) == lead) atomicAdd(&h[d0], (uint32_t)__popcll(m));
+    } else if (valid) {
+        atomicAdd(&h[d], 1u);
     }
+}
+
+// Morton code of box i: the scene box from the host (mn, ex) or, with `box`,
+// from the device: min xyz, max xyz, an empty extent taken as 1.
+struct Scene {
+    float mn0, mn1, mn2, ex0, ex1, ex2;
+    const float* box;
+};
+__device__ __forceinline__ Scene scene_of(Scene sc) {
+    if (sc.box) {
+        const float* box = sc.box;
+        sc.mn0 = box[0]; sc.mn1 = box[1]; sc.mn2 = box[2];
+        sc.ex0 = box[3] - sc.mn0; sc.ex1 = box[4] - sc.mn1; sc.ex2 = box[5] - sc.mn2;
+        sc.ex0 = sc.ex0 > 0.0f ? sc.ex0 : 1.0f; sc.ex1 = sc.ex1 > 0.0f ? sc.ex1 : 1.0f;
+        sc.ex2 = sc.ex2 > 0.0f ? sc.ex2 : 1.0f;
+    }
+    return sc;
+}
+__device__ __forceinline__ u64 morton_key(const float* __restrict__ aabbs, uint32_t i, const Scene& sc) {
     const float* b = aabbs + (size_t)i * 6u;
     const float cx = (b[0] + b[3]) * 0.5f, cy = (b[1] + b[4]) * 0.5f, cz = (b[2] + b[5]) * 0.5f;
-    code[i] = morton30((cx - mn0) / ex0, (cy - mn1) / ex1, (cz - mn2) / ex2);
-    idx[i] = i;
+    const uint32_t code = morton30((cx - sc.mn0) / sc.ex0, (cy - sc.mn1) / sc.ex1, (cz - sc.mn2) / sc.ex2);
+    return ((u64)code << 32) | (u64)i;
 }
 
-// ---- radix sort: histogram, scan, stable scatter (8-bit digits) ----
-__global__ void __launch_bounds__(kThreads) k_hist(const uint32_t* __restrict__ code, uint32_t n, const uint32_t* nd,
-                                                   uint32_t shift, uint32_t* __restrict__ hist, uint32_t nblocks) {
-    __shared__ uint32_t h[256];
+// ---- radix sort: stable, 8-bit digits, one launch per pass ----
+// Keys of all leaves, and each workgroup's histograms of the four digits
+// (rows[block][pass * 256 + digit]). Also clears what the sweeps share: the
+// tile tickets and, per pass, tile and digit, the status words.
+__global__ void __launch_bounds__(kThreads) k_morton(const float* __restrict__ aabbs, uint32_t n, const uint32_t* nd,
+                                                     Scene scene, u64* __restrict__ keys, uint32_t* __restrict__ rows,
+                                                     u64* __restrict__ status, uint32_t nstatus,
+                                                     uint32_t* __restrict__ tickets) {
+    __shared__ uint32_t h[kPasses * kDigits];
     n = leaf_count(n, nd);
-    const uint32_t base = blockIdx.x * kTile;
-    if (base >= n) {                          // tile past the leaves: an empty histogram
-        hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = 0u;
-        return;
-    }
-    h[threadIdx.x] = 0u;
+    h[threadIdx.x] = 0u;                       // kPasses * kDigits == kThreads
+    if (blockIdx.x == 0u && threadIdx.x < kPasses) tickets[threadIdx.x] = 0u;
+    for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < nstatus; i += gridDim.x * kThreads) status[i] = 0ull;
     __syncthreads();
-    for (uint32_t it = 0; it < kItems; ++it) {
-        const uint32_t i = base + it * kThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(code[i] >> shift) & 0xFFu], 1u);
+    const Scene sc = scene_of(scene);
+    for (uint32_t base = blockIdx.x * kThreads; base < n; base += gridDim.x * kThreads) {
+        const uint32_t i = base + threadIdx.x;
+        const bool valid = i < n;
+        u64 key = 0ull;
+        if (valid) {
+            key = morton_key(aabbs, i, sc);
+            keys[i] = key;
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < kPasses; ++p)
+            hist_add(h + p * kDigits, (uint32_t)(key >> (32u + 8u * p)) & 0xFFu, valid);
     }
     __syncthreads();
-    hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];   // digit-major
+    rows[(size_t)blockIdx.x * kThreads + threadIdx.x] = h[threadIdx.x];
+}
+static_assert(kPasses * kDigits == kThreads, "one histogram word per thread");
+
+// totals[pass * 256 + digit]: the histogram rows summed; a workgroup takes 64
+// columns, 16 row groups side by side.
+__global__ void __launch_bounds__(kThreads) k_digit_totals(const uint32_t* __restrict__ rows, uint32_t nrows,
+                                                           uint32_t* __restrict__ totals) {
+    __shared__ uint32_t part[kWaves][64];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t col = blockIdx.x * 64u + lane;
+    uint32_t s = 0;
+#pragma unroll 8
+    for (uint32_t r = w; r < nrows; r += kWaves) s += rows[(size_t)r * kThreads + col];
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0u) {
+        for (uint32_t k = 1; k < kWaves; ++k) s += part[k][lane];
+        totals[col] = s;
+    }
 }
 
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* sh, uint32_t* total) {
-    // 256 threads, 4 waves: wave inclusive scan by shuffles, then wave offsets
+struct SortLDS {
+    u64 key[kTile];                     // the tile in the order of this pass's digit
+    uint32_t wave[kWaves][kDigits];     // per wave: count, then offset of each digit
+    uint32_t first[kDigits];            // tile position of each digit's first key
+    uint32_t base[kDigits];             // output position of each digit's first key, less `first`
+    uint32_t sums[8];
+    uint32_t tile;
+};
+
+// Exclusive prefix over the first 256 threads (four waves; `sums` holds a
+// word per wave). Every thread of the workgroup calls it.
+__device__ __forceinline__ uint32_t scan256(uint32_t v, uint32_t* sums) {
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
     uint32_t x = v;
 #pragma unroll
@@ -227,191 +292,182 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
         const uint32_t y = __shfl_up(x, d);
         if ((int)lane >= d) x += y;
     }
-    if (lane == 63u) sh[w] = x;
+    if (w < 4u && lane == 63u) sums[w] = x;
     __syncthreads();
     uint32_t off = 0;
-    for (uint32_t k = 0; k < w; ++k) off += sh[k];
-    *total = sh[0] + sh[1] + sh[2] + sh[3];
+    for (uint32_t k = 0; k < 4u; ++k) off += k < w ? sums[k] : 0u;
     __syncthreads();
     return off + x - v;
 }
 
-__global__ void __launch_bounds__(kThreads) k_scan_reduce(const uint32_t* __restrict__ a, uint32_t n,
-                                                          uint32_t* __restrict__ part) {
-    __shared__ uint32_t sh[4];
-    const uint32_t base = blockIdx.x * kScanTile;
-    uint32_t s = 0;
-    for (uint32_t k = threadIdx.x; k < kScanTile; k += kThreads) {
-        const uint32_t i = base + k;
-        if (i < n) s += a[i];
-    }
-    uint32_t total;
-    (void)block_exclusive_scan(s, sh, &total);
-    if (threadIdx.x == 0) part[blockIdx.x] = total;
-}
-
-__global__ void __launch_bounds__(kThreads) k_scan_top(uint32_t* part, uint32_t nparts) {
-    __shared__ uint32_t sh[4];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nparts; base += kThreads) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < nparts ? part[i] : 0u;
-        uint32_t total;
-        const uint32_t ex = block_exclusive_scan(v, sh, &total);
-        if (i < nparts) part[i] = carry + ex;
-        carry += total;
-    }
-}
-
-__global__ void __launch_bounds__(kThreads) k_scan_down(uint32_t* __restrict__ a, uint32_t n,
-                                                        const uint32_t* __restrict__ part) {
-    __shared__ uint32_t sh[4];
-    const uint32_t base = blockIdx.x * kScanTile;
-    uint32_t carry = part[blockIdx.x];
-    for (uint32_t k = 0; k < kScanTile; k += kThreads) {
-        const uint32_t i = base + k + threadIdx.x;
-        const uint32_t v = i < n ? a[i] : 0u;
-        uint32_t total;
-        const uint32_t ex = block_exclusive_scan(v, sh, &total);
-        if (i < n) a[i] = carry + ex;
-        carry += total;
-    }
-}
-
-// keys_out (the last pass): the sorted 64-bit keys (code << 32 | index)
-// instead of the code and index arrays
-__global__ void __launch_bounds__(kThreads) k_scatter(const uint32_t* __restrict__ code_in,
-                                                      const uint32_t* __restrict__ idx_in,
-                                                      uint32_t* __restrict__ code_out, uint32_t* __restrict__ idx_out,
-                                                      unsigned long long* __restrict__ keys_out,
-                                                      uint32_t n, const uint32_t* nd, uint32_t shift,
-                                                      const uint32_t* __restrict__ offs, uint32_t nblocks) {
-    __shared__ uint32_t base_d[256];
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[4][256];
-    n = leaf_count(n, nd);
-    if (blockIdx.x * kTile >= n) return;      // whole workgroup: no leaves in this tile
+// Ranks the tile's keys by the digit at `shift`: S.first (first tile position
+// of each digit), rank[] (position of each key in the tile); thread d < 256
+// returns the tile's count of digit d. Wave w holds the keys w * 256 ..
+// w * 256 + 255 in tile order, 64 a step: within a step a lane's rank among
+// the lanes of its digit comes from eight ballots, and the wave's running
+// counts are its own, so the four steps need no barrier.
+__device__ __forceinline__ uint32_t rank_tile(SortLDS& S, const u64 key[kItems], uint32_t nvalid, uint32_t shift,
+                                              uint32_t rank[kItems]) {
     const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
-    base_d[t] = offs[(size_t)t * nblocks + blockIdx.x];
-    run[t] = 0u;
-    for (int k = 0; k < 4; ++k) wcnt[k][t] = 0u;
-    __syncthreads();
-    const unsigned long long lt = (1ull << lane) - 1ull;
+    // LDS pointer of its own address space: volatile accesses through a generic
+    // one would be flat loads and stores
+    typedef __attribute__((address_space(3))) volatile uint32_t lds_u32;
+    lds_u32* mine = (lds_u32*)S.wave[w];
+    for (uint32_t k = lane; k < kDigits; k += 64u) mine[k] = 0u;
+    const u64 lt = (1ull << lane) - 1ull;
+#pragma unroll
     for (uint32_t it = 0; it < kItems; ++it) {
-        const uint32_t i = blockIdx.x * kTile + it * kThreads + t;
-        const bool valid = i < n;
-        const uint32_t key = valid ? code_in[i] : 0u;
-        const uint32_t val = valid ? idx_in[i] : 0u;
-        const uint32_t d = (key >> shift) & 0xFFu;
-        // lanes of this wave holding the same digit
-        unsigned long long peers = __ballot(valid);
+        const bool valid = w * 256u + it * 64u + lane < nvalid;
+        const uint32_t d = (uint32_t)(key[it] >> shift) & 0xFFu;
+        u64 peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
-            const unsigned long long on = __ballot(valid && ((d >> b) & 1u));
+            const u64 on = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? on : ~on;
         }
-        const uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0u) wcnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t off = base_d[d] + run[d] + rank;
-            for (uint32_t k = 0; k < w; ++k) off += wcnt[k][d];
-            if (off < n) {            // always true when the histograms are consistent
-                if (keys_out) {
-                    keys_out[off] = ((unsigned long long)key << 32) | (unsigned long long)val;
-                } else {
-                    code_out[off] = key;
-                    idx_out[off] = val;
-                }
-            }
-        }
-        __syncthreads();
-        run[t] += wcnt[0][t] + wcnt[1][t] + wcnt[2][t] + wcnt[3][t];
-        for (int k = 0; k < 4; ++k) wcnt[k][t] = 0u;
-        __syncthreads();
-    }
-}
-
-// ---- Karras build ----
-// The keys of the workgroup's nodes and kKarrasHalo keys on either side are
-// staged in LDS: most nodes span few leaves, so their searches stay in the
-// window; a search that leaves it reads the key from global memory.
-constexpr int kKarrasHalo = 256;
-constexpr int kKarrasWindow = 256 + 2 * kKarrasHalo;
-
-// other_end[i]: the end of node i's leaf range other than i (the range is
-// [min(i, j), max(i, j)])
-__global__ void __launch_bounds__(256) k_karras(const unsigned long long* __restrict__ keys, uint32_t n,
-                                                const uint32_t* nd, int32_t* __restrict__ left,
-                                                int32_t* __restrict__ right, int32_t* __restrict__ parent,
-                                                int32_t* __restrict__ leaf_parent, int32_t* __restrict__ other_end,
-                                                uint32_t* __restrict__ ticket) {
-    __shared__ unsigned long long sk[kKarrasWindow];
-    const int64_t nn = leaf_count(n, nd);
-    const int64_t ws = (int64_t)blockIdx.x * blockDim.x - kKarrasHalo;
-    for (int t = threadIdx.x; t < kKarrasWindow; t += blockDim.x) {
-        const int64_t k = ws + t;
-        sk[t] = (k >= 0 && k < nn) ? keys[k] : 0ull;
+        const uint32_t before = mine[d], r = (uint32_t)__popcll(peers & lt);
+        __builtin_amdgcn_wave_barrier();       // every lane has read the count its digit had
+        if (valid && r == 0u) mine[d] = before + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        rank[it] = before + r;
     }
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nn - 1) return;
-    ticket[i] = 0u;
-    if (i == 0) parent[0] = -1;
-    // LDS and global pointers of their own address spaces: the two loads
-    // cannot be merged into one load through a selected generic pointer,
-    // which would be a flat load
-    typedef __attribute__((address_space(3))) const unsigned long long lds_u64;
-    typedef __attribute__((address_space(1))) const unsigned long long glb_u64;
-    const lds_u64* wk = (const lds_u64*)sk;
-    const glb_u64* gk = (const glb_u64*)keys;
-    const unsigned long long ki = wk[i - ws];
-    auto delta = [&](int64_t jj) -> int {
-        if (jj < 0 || jj >= nn) return -1;
-        const int64_t o = jj - ws;
-        unsigned long long kj;
-        if (o >= 0 && o < kKarrasWindow) kj = wk[o];
-        else kj = gk[jj];
-        return __clzll((long long)(ki ^ kj));
-    };
-    const int dir = (delta(i + 1) - delta(i - 1)) >= 0 ? 1 : -1;
-    const int dmin = delta(i - dir);
-    int64_t lmax = 2;
-    while (delta(i + lmax * dir) > dmin) lmax *= 2;
-    int64_t l = 0;
-    for (int64_t t = lmax / 2; t >= 1; t /= 2)
-        if (delta(i + (l + t) * dir) > dmin) l += t;
-    const int64_t j = i + l * dir;
-    const int dnode = delta(j);
-    int64_t s = 0;
-    for (int64_t t = (l + 1) / 2;; t = (t + 1) / 2) {
-        if (delta(i + (s + t) * dir) > dnode) s += t;
-        if (t == 1) break;
+    uint32_t total = 0;
+    if (t < kDigits)
+        for (uint32_t k = 0; k < kWaves; ++k) {
+            const uint32_t c = S.wave[k][t];
+            S.wave[k][t] = total;
+            total += c;
+        }
+    const uint32_t f = scan256(total, S.sums);
+    if (t < kDigits) S.first[t] = f;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t it = 0; it < kItems; ++it) {
+        const uint32_t d = (uint32_t)(key[it] >> shift) & 0xFFu;
+        rank[it] += S.first[d] + S.wave[w][d];
     }
-    const int64_t gamma = i + s * dir + (dir < 0 ? -1 : 0);
-    const int32_t lc = (min(i, j) == gamma) ? (int32_t)gamma : -(int32_t)gamma;
-    const int32_t rc = (max(i, j) == gamma + 1) ? (int32_t)(gamma + 1) : -(int32_t)(gamma + 1);
-    left[i] = lc;
-    right[i] = rc;
-    other_end[i] = (int32_t)j;
-    if (lc < 0) parent[-lc] = (int32_t)i; else leaf_parent[lc] = (int32_t)i;
-    if (rc < 0) parent[-rc] = (int32_t)i; else leaf_parent[rc] = (int32_t)i;
+    return total;
 }
 
-// ---- refit ----
-__device__ __forceinline__ void store_box(float* p, const float b[6]) {
+// Status words of the look-back: the tile's count of a digit (kCount), or
+// with all tiles before it (kPrefix), in the low 62 bits. One 64-bit word
+// carries flag and value, so relaxed agent-scope accesses order themselves.
+constexpr u64 kCount = 1ull << 62, kPrefix = 2ull << 62, kValue = (1ull << 62) - 1ull;
+
+// One pass: the tile's keys ranked in LDS, the tile's place in the output of
+// every digit found by looking back over the tiles before it, the keys
+// written in tile order (runs of consecutive keys per digit). A tile waits
+// for lower tiles only, and tiles are numbered by ticket in the order in
+// which workgroups start, so the lowest unfinished tile is always running and
+// never waits: every wait ends. The look-back reads eight tiles at a time:
+// their words are independent loads, and one at a time the tiles of a million
+// keys would be a chain of up to 245 round trips to memory. A million keys
+// sort in 4 x 16.7 us; a histogram, three scan launches and a scatter a pass
+// took 181 us (20 launches).
+__global__ void __launch_bounds__(kThreads) k_sweep(const u64* __restrict__ in, u64* __restrict__ out, uint32_t n,
+                                                    const uint32_t* nd, uint32_t pass,
+                                                    const uint32_t* __restrict__ totals, u64* status,
+                                                    uint32_t* tickets) {
+    __shared__ SortLDS S;
+    n = leaf_count(n, nd);
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6, shift = 32u + 8u * pass;
+    if (t == 0u) S.tile = atomicAdd(&tickets[pass], 1u);
+    __syncthreads();
+    const uint32_t tile = S.tile;
+    if ((uint64_t)tile * kTile >= n) return;            // whole workgroup: no keys here
+    const uint32_t s = tile * kTile, cnt = min(kTile, n - s);
+    u64 key[kItems];
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
-        __hip_atomic_store(reinterpret_cast<uint32_t*>(p) + q, __float_as_uint(b[q]), __ATOMIC_RELAXED,
+    for (uint32_t it = 0; it < kItems; ++it) {
+        const uint32_t q = w * 256u + it * 64u + lane;
+        key[it] = q < cnt ? in[s + q] : 0ull;
+    }
+    uint32_t rank[kItems];
+    const uint32_t total = rank_tile(S, key, cnt, shift, rank);
+    u64* st = status + t;                               // word of tile k: st[k * 256]
+    if (t < kDigits)
+        __hip_atomic_store(&st[(size_t)tile * kDigits], (tile ? kCount : kPrefix) | total, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void load_box(const float* p, float b[6]) {
 #pragma unroll
-    for (int q = 0; q < 6; ++q)
-        b[q] = __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(p) + q, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT));
+    for (uint32_t it = 0; it < kItems; ++it)
+        if (w * 256u + it * 64u + lane < cnt) S.key[rank[it]] = key[it];
+    const uint32_t g = scan256(t < kDigits ? totals[pass * kDigits + t] : 0u, S.sums);
+    if (t < kDigits) {
+        uint32_t before = 0;
+        int64_t k = (int64_t)tile - 1;                  // the nearest tile not yet added
+        constexpr int kBack = 8;
+        while (k >= 0) {
+            u64 v[kBack];
+#pragma unroll
+            for (int b = 0; b < kBack; ++b)
+                v[b] = __hip_atomic_load(&st[(size_t)(k - b > 0 ? k - b : 0) * kDigits], __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+            bool open = true;                           // every nearer word has been there
+#pragma unroll
+            for (int b = 0; b < kBack; ++b) {
+                if (!open || k < 0) continue;
+                if (v[b] < kCount) { open = false; continue; }
+                before += (uint32_t)(v[b] & kValue);
+                k = v[b] >= kPrefix ? -1 : k - 1;
+            }
+            if (!open) __builtin_amdgcn_s_sleep(1);
+        }
+        if (tile)
+            __hip_atomic_store(&st[(size_t)tile * kDigits], kPrefix | (u64)(before + total), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        S.base[t] = g + before - S.first[t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t it = 0; it < kItems; ++it) {
+        const uint32_t q = it * kThreads + t;
+        if (q < cnt) {
+            const u64 x = S.key[q];
+            const uint32_t off = S.base[(uint32_t)(x >> shift) & 0xFFu] + q;
+            if (off < n) out[off] = x;                  // always true: the totals count these keys
+        }
+    }
 }
 
+// Up to kSmallLeaves leaves (one sort tile): keys and sort in one workgroup,
+// 17.8 us for 3,001 leaves, where the launches above would take about 45 us
+// (9 us a pass at a few tiles) and the separate scans took 120.
+__global__ void __launch_bounds__(kThreads) k_sort_small(const float* __restrict__ aabbs, uint32_t n,
+                                                         const uint32_t* nd, Scene scene, u64* __restrict__ keys) {
+    __shared__ SortLDS S;
+    n = min(leaf_count(n, nd), kSmallLeaves);
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    const Scene sc = scene_of(scene);
+    u64 key[kItems];
+#pragma unroll
+    for (uint32_t it = 0; it < kItems; ++it) {
+        const uint32_t i = w * 256u + it * 64u + lane;
+        key[it] = i < n ? morton_key(aabbs, i, sc) : 0ull;
+    }
+#pragma unroll 1
+    for (uint32_t pass = 0; pass < kPasses; ++pass) {
+        uint32_t rank[kItems];
+        (void)rank_tile(S, key, n, 32u + 8u * pass, rank);
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it)
+            if (w * 256u + it * 64u + lane < n) S.key[rank[it]] = key[it];
+        __syncthreads();
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it) {
+            const uint32_t i = w * 256u + it * 64u + lane;
+            if (i < n) key[it] = S.key[i];
+        }
+        // the next pass writes S.key after its barriers
+    }
+#pragma unroll
+    for (uint32_t it = 0; it < kItems; ++it) {
+        const uint32_t i = w * 256u + it * 64u + lane;
+        if (i < n) keys[i] = key[it];
+    }
+}
+
+// ---- the tree ----
 // The union is taken in child order, left box first: min(L, R) = R < L ? R : L
 // and max(L, R) = L < R ? R : L, as std::min / std::max fold them.
 __device__ __forceinline__ void unite(const float b[6], const float o[6], bool mine_left, float u[6]) {
@@ -422,199 +478,295 @@ __device__ __forceinline__ void unite(const float b[6], const float o[6], bool m
     }
 }
 
-// a node is local to the tile [s, e) of sorted leaves when its leaf range
-// [min(i, j), max(i, j)] lies inside it; both its children then do too
-__device__ __forceinline__ bool is_local(int32_t i, int32_t j, uint32_t s, uint32_t e) {
-    return (uint32_t)min(i, j) >= s && (uint32_t)max(i, j) < e;
-}
-__device__ __forceinline__ uint32_t tile_of(uint32_t leaf) { return leaf / kRefitTile; }
+struct TreeOut {
+    int32_t *left, *right, *parent, *leaf_parent;
+    int32_t* other_end;                 // the end of node i's leaf range other than i (NULL: not wanted)
+    float* node_aabb;
+};
 
-// Refit, first kernel: one workgroup per tile of kRefitTile sorted leaves
-// completes the tile's local nodes. A local node's index lies in its own
-// range, so in the tile: the tile's topology (children, parent, range end,
-// leaf parents) and leaf boxes are staged in LDS with coalesced loads, and
-// both climbing threads of a local node belong to the workgroup, so its ticket
-// and box live in LDS too. A climb stops where it
-// would enter a node spanning tiles; the second kernel starts there. Every
-// completed box goes to node_aabb with plain stores, which the next kernel
-// sees.
-__global__ void __launch_bounds__(256) k_refit_local(const float* __restrict__ aabbs,
-                                                     const unsigned long long* __restrict__ keys, uint32_t n,
-                                                     const uint32_t* nd, const int32_t* __restrict__ left,
-                                                     const int32_t* __restrict__ right,
-                                                     const int32_t* __restrict__ parent,
-                                                     const int32_t* __restrict__ leaf_parent,
-                                                     const int32_t* __restrict__ other_end,
-                                                     float* __restrict__ node_aabb) {
-    __shared__ __align__(16) float lbox[kRefitTile * 6];   // the tile's leaf boxes, sorted order
-    __shared__ float nbox[kRefitTile * 6];    // boxes of the tile's local nodes (index - s)
-    __shared__ uint32_t ltk[kRefitTile];      // tickets of the tile's local nodes
-    __shared__ int32_t tl[kRefitTile], tr[kRefitTile], tp[kRefitTile], te[kRefitTile], tlp[kRefitTile];
-    n = leaf_count(n, nd);
-    const uint32_t s = blockIdx.x * kRefitTile;
-    if (n < 2u || s >= n) return;             // one leaf: no internal node, no parent links
-    const uint32_t e = min(s + kRefitTile, n);
-    // staging: every load of a thread's slots is issued before any is waited
-    // for. Indices are clamped into range so that the loads need no branch;
-    // validity only selects what is stored. Leaf boxes are gathered through
-    // the sorted keys, 8 bytes at a time (boxes are 24-byte records).
-    constexpr uint32_t kSlots = kRefitTile / 256u;
-    const uint32_t last_leaf = e - 1u, last_node = n - 2u;
-    uint32_t box_of[kSlots];
-#pragma unroll
-    for (uint32_t u = 0; u < kSlots; ++u)
-        box_of[u] = (uint32_t)(keys[min(s + threadIdx.x + u * 256u, last_leaf)] & 0xFFFFFFFFull);
-    float2 gb[kSlots][3];
-    int32_t vlp[kSlots], vl[kSlots], vr[kSlots], vp[kSlots], ve[kSlots];
-#pragma unroll
-    for (uint32_t u = 0; u < kSlots; ++u) {
-        const uint32_t i = s + threadIdx.x + u * 256u;
-        const float2* src = reinterpret_cast<const float2*>(aabbs + (size_t)box_of[u] * 6u);
-        gb[u][0] = src[0];
-        gb[u][1] = src[1];
-        gb[u][2] = src[2];
-        const uint32_t li = min(i, last_leaf), ni = min(i, last_node);
-        vlp[u] = leaf_parent[li];
-        vl[u] = left[ni];
-        vr[u] = right[ni];
-        vp[u] = parent[ni];
-        ve[u] = other_end[ni];
+// A subtree over the sorted leaves [l, r] whose parent reaches beyond the
+// workgroup that completed it, with its box.
+struct __align__(16) Root {
+    uint32_t l, r;
+    float2 b0, b1, b2;
+};
+
+// The items of a workgroup, in leaf order: leaves (CAP = kTreeTile), or the
+// open subtrees of the level before (CAP = kTreeGroup * kMaxRoots).
+template <uint32_t CAP>
+struct TreeLDS {
+    float2 box[CAP * 3u];               // the box a subtree left for its sibling, at the end the sibling meets
+    uint32_t slot[CAP];                 // split between items q and q + 1: the far end (+ 1) of the child that came first
+    uint16_t mark[CAP];                 // open subtree starting at item q: its end + 1 | 0x8000 for a right child
+    int8_t delta[CAP + 4u];             // common prefix of the keys either side of item q's start (-1: none)
+    uint32_t sums[kWaves];
+};
+// ... and what the first level writes out at the end, by tile position
+struct LeafOut {
+    uint16_t node[kTreeTile];           // node: split | kLeftLeaf | kRightLeaf (kNoNode: made elsewhere)
+    uint16_t parent[kTreeTile];         // parent of node / leaf (kNoNode: made elsewhere)
+    uint16_t leaf_parent[kTreeTile];
+    uint16_t other_end[kTreeTile];
+};
+constexpr uint32_t kLeftLeaf = 0x4000u, kRightLeaf = 0x8000u, kNoNode = 0xFFFFu;   // split < kTreeTile <= 0x4000
+// ... and the first leaf of each item above it ([m]: the leaf after the last item)
+struct RootIn {
+    uint32_t first[kTreeGroup * kMaxRoots + 1u];
+    uint32_t pre[kTreeGroup + 1u];
+};
+
+// Common prefix length of the keys of leaves x - 1 and x, -1 at the ends.
+__device__ __forceinline__ int key_delta(const u64* __restrict__ keys, uint32_t x, uint32_t n) {
+    return x == 0u || x >= n ? -1 : __clzll((long long)(keys[x - 1u] ^ keys[x]));
+}
+
+// Climbs from item q with box b until the sibling has not come yet, the
+// parent reaches beyond the workgroup's m items (mark), or the root is done.
+// A subtree [ql, qr] is the right child of its parent when its first key
+// shares more bits with the key before it than its last with the key after
+// it; the two are never equal, as the keys are unique. Both children meet at
+// the split between them. A subtree leaves its box at its end next to the
+// split, before the exchange of the slot: two subtrees with that end are
+// nested, and the inner one's box was taken before the outer one existed.
+// That end is the subtree's node number, so at the end box[] holds the boxes
+// of the nodes made here.
+// The climb is a chain of LDS round trips (the exchange, then the sibling's
+// box and the key distance at its far end), at two workgroups of 16 waves a
+// compute unit. The first level's nodes go out afterwards, in order, instead
+// of seven scattered stores a step with a few lanes left: k_tree_leaves over
+// a million leaves 53 -> 45 us. A Karras search per node and a separate refit
+// through global memory (three kernels, which read the topology back) took
+// 142 us for what the levels here do in 45 + 46.
+template <bool LEAVES, uint32_t CAP>
+__device__ __forceinline__ void climb(TreeLDS<CAP>& T, LeafOut* lo, const RootIn* in, const TreeOut& out, uint32_t m,
+                                      uint32_t q, float2 b0, float2 b1, float2 b2) {
+    uint32_t ql = q, qr = q;
+    uint32_t L = LEAVES ? q : in->first[q], R1 = LEAVES ? q + 1u : in->first[q + 1u];   // leaves [L, R1)
+    int dl = T.delta[ql], dr = T.delta[qr + 1u];
+    bool made = false;                  // [ql, qr] is a node made here: split before leaf P, children leaves or nodes
+    uint32_t P = 0;
+    bool lleaf = false, rleaf = false;
+    for (;;) {
+        const bool root = dl < 0 && dr < 0, right = dl > dr;
+        if (made) {
+            const uint32_t node = root ? 0u : (right ? L : R1 - 1u);
+            if (LEAVES) {
+                lo->node[node] = (uint16_t)((P - 1u) | (lleaf ? kLeftLeaf : 0u) | (rleaf ? kRightLeaf : 0u));
+                uint16_t* pl = lleaf ? lo->leaf_parent : lo->parent;
+                uint16_t* pr = rleaf ? lo->leaf_parent : lo->parent;
+                pl[P - 1u] = (uint16_t)node;
+                pr[P] = (uint16_t)node;
+                lo->other_end[node] = (uint16_t)(node == L ? R1 - 1u : L);
+            } else {
+                const int32_t lc = lleaf ? (int32_t)(P - 1u) : -(int32_t)(P - 1u), rc = rleaf ? (int32_t)P : -(int32_t)P;
+                out.left[node] = lc;
+                out.right[node] = rc;
+                (lleaf ? out.leaf_parent : out.parent)[P - 1u] = (int32_t)node;
+                (rleaf ? out.leaf_parent : out.parent)[P] = (int32_t)node;
+                if (root) out.parent[0] = -1;
+                if (out.other_end) out.other_end[node] = (int32_t)(node == L ? R1 - 1u : L);
+                box2* o = reinterpret_cast<box2*>(out.node_aabb + (size_t)node * 6u);
+                o[0] = box2{b0.x, b0.y};
+                o[1] = box2{b1.x, b1.y};
+                o[2] = box2{b2.x, b2.y};
+            }
+        }
+        float2* mine = &T.box[(root ? 0u : (right ? ql : qr)) * 3u];
+        mine[0] = b0;
+        mine[1] = b1;
+        mine[2] = b2;
+        if (root) return;
+        if (right ? ql == 0u : qr + 1u == m) {
+            T.mark[ql] = (uint16_t)((qr + 1u) | (right ? 0x8000u : 0u));
+            return;
+        }
+        const uint32_t sp = right ? ql - 1u : qr;
+        // only LDS needs ordering: the box is in place before the slot is
+        // exchanged, and the sibling's is read after it
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const uint32_t v = __hip_atomic_exchange(&T.slot[sp], (right ? qr : ql) + 1u, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+        asm volatile("" ::: "memory");
+        if (v == 0u) return;            // the sibling's thread goes on from here
+        T.slot[sp] = 0u;                // both have come
+        const float2* src = &T.box[(right ? sp : sp + 1u) * 3u];
+        const float2 s0 = src[0], s1 = src[1], s2 = src[2];
+        const uint32_t far = v - 1u;    // the sibling's far end
+        const int d = T.delta[right ? far : far + 1u];
+        const uint32_t F = LEAVES ? (right ? far : far + 1u) : in->first[right ? far : far + 1u];
+        const float bb[6] = {b0.x, b0.y, b1.x, b1.y, b2.x, b2.y}, o[6] = {s0.x, s0.y, s1.x, s1.y, s2.x, s2.y};
+        float u[6];
+        unite(bb, o, !right, u);
+        b0 = make_float2(u[0], u[1]);
+        b1 = make_float2(u[2], u[3]);
+        b2 = make_float2(u[4], u[5]);
+        if (right) {
+            P = L;
+            rleaf = R1 - L == 1u;
+            lleaf = L - F == 1u;
+            L = F; ql = far; dl = d;
+        } else {
+            P = R1;
+            lleaf = R1 - L == 1u;
+            rleaf = F - R1 == 1u;
+            R1 = F; qr = far; dr = d;
+        }
+        made = true;
     }
-#pragma unroll
-    for (uint32_t u = 0; u < kSlots; ++u) {
-        const uint32_t k = threadIdx.x + u * 256u, i = s + k;
-        const bool internal = i < e && i <= last_node;   // internal nodes 0 .. n-2
-        ltk[k] = 0u;
-        tlp[k] = vlp[u];
-        tl[k] = vl[u];
-        tr[k] = vr[u];
-        tp[k] = vp[u];
-        te[k] = internal ? ve[u] : -1;                   // -1: never local
-        float2* d = reinterpret_cast<float2*>(&lbox[k * 6u]);
-        d[0] = gb[u][0];
-        d[1] = gb[u][1];
-        d[2] = gb[u][2];
+}
+
+// The open subtrees of the workgroup, in leaf order: those marked, and those
+// whose sibling has not come to their split. Every thread calls it after all
+// climbs. A level's roots are at most kMaxRoots: they are the siblings that
+// hang off the two paths from the tree's root to the workgroup's first and
+// last leaf, and a radix tree over unique 64-bit keys whose top two bits are
+// zero is at most 62 levels deep.
+template <uint32_t CAP>
+__device__ __forceinline__ void leave_roots(TreeLDS<CAP>& T, const RootIn* in, uint32_t s, uint32_t m,
+                                            Root* __restrict__ roots, uint32_t* __restrict__ nroots) {
+    constexpr uint32_t K = CAP / kThreads;      // in: first leaves of the items (NULL: item q is leaf s + q)
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    __syncthreads();
+    for (uint32_t q = t; q < m; q += kThreads) {
+        const uint32_t v = T.slot[q];
+        if (v == 0u) continue;
+        if (v - 1u <= q) T.mark[v - 1u] = (uint16_t)(q + 1u);      // the left child [v - 1, q]
+        else T.mark[q + 1u] = (uint16_t)(v | 0x8000u);             // the right child [q + 1, v - 1]
     }
     __syncthreads();
-    for (uint32_t k = s + threadIdx.x; k < e; k += blockDim.x) {
-        float b[6];
+    uint32_t c = 0;
 #pragma unroll
-        for (int q = 0; q < 6; ++q) b[q] = lbox[(k - s) * 6u + q];
-        int32_t cur = (int32_t)k;             // leaf k, or the local node just completed
-        bool cur_leaf = true;
-        int32_t node = tlp[k - s];
-        // a radix tree over unique 64-bit keys is at most 65 levels deep
-        for (int guard = 0; node >= 0 && guard < 96; ++guard) {
-            if ((uint32_t)node < s || (uint32_t)node >= e) break;   // outside the tile: spanning
-            const uint32_t x = (uint32_t)node - s;
-            const int32_t j = te[x];
-            if (j < 0 || !is_local(node, j, s, e)) break;
-            // only LDS needs ordering here: this thread's LDS box writes are
-            // complete before its ticket, and the sibling's box is read after
-            // it (a release at workgroup scope would also wait for the global
-            // stores of node_aabb)
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const uint32_t t = __hip_atomic_fetch_add(&ltk[x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            asm volatile("" ::: "memory");
-            if (t == 0u) break;               // the sibling's thread finishes this node
-            const int32_t l = tl[x], r = tr[x];
-            const bool mine_left = cur_leaf ? (l == cur) : (l == -cur);
-            const int32_t sib = mine_left ? r : l;
-            const float* src = sib >= 0 ? &lbox[(uint32_t)(sib - (int32_t)s) * 6u]
-                                        : &nbox[(uint32_t)(-sib - (int32_t)s) * 6u];
-            float o[6], u[6];
+    for (uint32_t k = 0; k < K; ++k) c += t * K + k < m && T.mark[t * K + k] != 0u ? 1u : 0u;
+    uint32_t x = c;
 #pragma unroll
-            for (int q = 0; q < 6; ++q) o[q] = src[q];
-            unite(b, o, mine_left, u);
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d);
+        if ((int)lane >= d) x += y;
+    }
+    if (lane == 63u) T.sums[w] = x;
+    __syncthreads();
+    uint32_t off = x - c, all = 0;
+    for (uint32_t k = 0; k < kWaves; ++k) {
+        off += k < w ? T.sums[k] : 0u;
+        all += T.sums[k];
+    }
+    if (t == 0u) *nroots = min(all, kMaxRoots);
 #pragma unroll
-            for (int q = 0; q < 6; ++q) {
-                b[q] = u[q];
-                nbox[x * 6u + q] = u[q];
-                node_aabb[(size_t)node * 6u + q] = u[q];
-            }
-            cur = node;
-            cur_leaf = false;
-            if (node == 0) break;
-            node = tp[x];
+    for (uint32_t k = 0; k < K; ++k) {
+        const uint32_t q = t * K + k;
+        if (q >= m || T.mark[q] == 0u) continue;
+        const uint32_t e = T.mark[q] & 0x7FFFu, at = (T.mark[q] & 0x8000u) ? q : e - 1u;
+        if (off < kMaxRoots) {
+            Root r;
+            r.l = in ? in->first[q] : s + q;
+            r.r = (in ? in->first[e] : s + e) - 1u;
+            r.b0 = T.box[at * 3u];
+            r.b1 = T.box[at * 3u + 1u];
+            r.b2 = T.box[at * 3u + 2u];
+            roots[off] = r;
+        }
+        ++off;
+    }
+}
+
+// First level: a workgroup per tile of kTreeTile sorted leaves, one leaf per
+// thread (41 KB of LDS, two workgroups of 16 waves per compute unit). What
+// bounds it is the gather of the leaf boxes through the sorted keys (24 bytes
+// from a 128-byte line each) and the length of the climbs in LDS; the tile's
+// nodes are written in order afterwards.
+__global__ void __launch_bounds__(kThreads) k_tree_leaves(const float* __restrict__ aabbs,
+                                                          const u64* __restrict__ keys, uint32_t n, const uint32_t* nd,
+                                                          TreeOut out, Root* __restrict__ roots,
+                                                          uint32_t* __restrict__ nroots) {
+    __shared__ __align__(16) TreeLDS<kTreeTile> T;
+    __shared__ LeafOut O;
+    static_assert(kTreeTile == kThreads, "one leaf per thread");
+    n = leaf_count(n, nd);
+    const uint32_t q = threadIdx.x, s = blockIdx.x * kTreeTile;
+    if (s >= n) {
+        if (q == 0u) nroots[blockIdx.x] = 0u;
+        return;
+    }
+    const uint32_t m = min(kTreeTile, n - s);
+    const uint32_t i = s + min(q, m - 1u);
+    const u64 key = keys[i];
+    const box2* src = reinterpret_cast<const box2*>(aabbs + (size_t)(uint32_t)key * 6u);
+    const box2 g0 = src[0], g1 = src[1], g2 = src[2];
+    T.slot[q] = 0u;
+    T.mark[q] = 0u;
+    O.node[q] = O.parent[q] = O.leaf_parent[q] = (uint16_t)kNoNode;
+    if (q < m) T.delta[q] = (int8_t)(i == 0u ? -1 : __clzll((long long)(keys[i - 1u] ^ key)));
+    if (q == 0u) T.delta[m] = (int8_t)key_delta(keys, s + m, n);
+    __syncthreads();
+    if (q < m)
+        climb<true>(T, &O, nullptr, out, m, q, make_float2(g0.x, g0.y), make_float2(g1.x, g1.y),
+                    make_float2(g2.x, g2.y));
+    leave_roots(T, nullptr, s, m, roots + (size_t)blockIdx.x * kMaxRoots, nroots + blockIdx.x);
+    if (q >= m) return;
+    const uint32_t node = O.node[q], par = O.parent[q], lpar = O.leaf_parent[q];
+    if (lpar != kNoNode) out.leaf_parent[i] = (int32_t)(s + lpar);
+    if (par != kNoNode) out.parent[i] = (int32_t)(s + par);
+    if (node != kNoNode) {
+        const int32_t p = (int32_t)(s + (node & 0x3FFFu));
+        out.left[i] = (node & kLeftLeaf) ? p : -p;
+        out.right[i] = (node & kRightLeaf) ? p + 1 : -(p + 1);
+        if (out.other_end) out.other_end[i] = (int32_t)(s + O.other_end[q]);
+        box2* o = reinterpret_cast<box2*>(out.node_aabb + (size_t)i * 6u);
+        const float2 a = T.box[q * 3u], b = T.box[q * 3u + 1u], c = T.box[q * 3u + 2u];
+        o[0] = box2{a.x, a.y};
+        o[1] = box2{b.x, b.y};
+        o[2] = box2{c.x, c.y};
+        if (i == 0u) out.parent[0] = -1;        // the whole tree is one tile
+    }
+}
+
+// The levels above: a workgroup takes the open subtrees of kTreeGroup
+// workgroups of the level before.
+__global__ void __launch_bounds__(kThreads) k_tree_roots(const u64* __restrict__ keys, uint32_t n, const uint32_t* nd,
+                                                         TreeOut out, const Root* __restrict__ in,
+                                                         const uint32_t* __restrict__ nin, uint32_t groups,
+                                                         Root* __restrict__ roots, uint32_t* __restrict__ nroots) {
+    constexpr uint32_t CAP = kTreeGroup * kMaxRoots;
+    __shared__ __align__(16) TreeLDS<CAP> T;
+    __shared__ RootIn I;
+    n = leaf_count(n, nd);
+    const uint32_t t = threadIdx.x, g0 = blockIdx.x * kTreeGroup;
+    if (t < 64u) {                      // one wave: prefix of the groups' counts
+        const uint32_t c = t < kTreeGroup && g0 + t < groups ? min(nin[g0 + t], kMaxRoots) : 0u;
+        uint32_t x = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d);
+            if ((int)t >= d) x += y;
+        }
+        if (t <= kTreeGroup) I.pre[t] = x - c;
+    }
+    __syncthreads();
+    const uint32_t m = I.pre[kTreeGroup];
+    if (m == 0u) {
+        if (t == 0u) nroots[blockIdx.x] = 0u;
+        return;
+    }
+    for (uint32_t x = t; x < CAP; x += kThreads) {
+        const uint32_t c = x / kMaxRoots, q = I.pre[c] + x % kMaxRoots;
+        if (q >= I.pre[c + 1u]) continue;
+        const Root r = in[(size_t)g0 * kMaxRoots + x];
+        I.first[q] = r.l;
+        T.box[q * 3u] = r.b0;
+        T.box[q * 3u + 1u] = r.b1;
+        T.box[q * 3u + 2u] = r.b2;
+        T.delta[q] = (int8_t)key_delta(keys, r.l, n);
+        T.slot[q] = 0u;
+        T.mark[q] = 0u;
+        if (q + 1u == m) {
+            I.first[m] = r.r + 1u;
+            T.delta[m] = (int8_t)key_delta(keys, r.r + 1u, n);
         }
     }
-}
-
-// the box of child c of a node spanning tiles: a leaf's from the input, a
-// local node's as the first kernel left it
-__device__ __forceinline__ void child_box(const float* aabbs, const unsigned long long* keys, const float* node_aabb,
-                                          int32_t c, float o[6]) {
-    const float* src = c >= 0 ? aabbs + (size_t)(keys[c] & 0xFFFFFFFFull) * 6u : node_aabb + (size_t)(-c) * 6u;
-#pragma unroll
-    for (int q = 0; q < 6; ++q) o[q] = src[q];
-}
-
-// Refit, second kernel: the nodes spanning tiles. One thread per internal
-// node; a spanning node with a child that is a leaf or a local node (both
-// complete) starts a climb there - with both children complete it unites them
-// at once, with one it takes the node's ticket - and climbs as the reference
-// does: the first arriver stops, the second unites and goes on. Boxes that
-// climbs exchange are written and read with agent-scope atomics, each store
-// complete before the next ticket.
-__global__ void __launch_bounds__(256) k_refit_global(const float* __restrict__ aabbs,
-                                                      const unsigned long long* __restrict__ keys, uint32_t n,
-                                                      const uint32_t* nd, const int32_t* __restrict__ left,
-                                                      const int32_t* __restrict__ right,
-                                                      const int32_t* __restrict__ parent,
-                                                      const int32_t* __restrict__ other_end, float* node_aabb,
-                                                      uint32_t* ticket) {
-    n = leaf_count(n, nd);
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n < 2u || i >= n - 1u) return;
-    const int32_t node0 = (int32_t)i, j = other_end[i];
-    const uint32_t lo = (uint32_t)min(node0, j), hi = (uint32_t)max(node0, j);
-    if (tile_of(lo) == tile_of(hi)) return;   // local: done by the first kernel
-    const int32_t l = left[i], r = right[i];
-    // a child is complete when it is a leaf or a node inside one tile
-    auto complete = [&](int32_t c) {
-        if (c >= 0) return true;
-        const int32_t jj = other_end[-c];
-        return tile_of((uint32_t)min(-c, jj)) == tile_of((uint32_t)max(-c, jj));
-    };
-    const bool lc = complete(l), rc = complete(r);
-    if (!lc && !rc) return;                   // both children arrive by climbs
-    float b[6];
-    int32_t cur, node = node0;
-    if (lc && rc) {                           // both known: this node is complete now
-        float lb[6], rb[6];
-        child_box(aabbs, keys, node_aabb, l, lb);
-        child_box(aabbs, keys, node_aabb, r, rb);
-        unite(lb, rb, true, b);
-        store_box(node_aabb + (size_t)node * 6u, b);
-        if (node == 0) return;
-        cur = -node;
-        node = parent[node];
-    } else {
-        cur = lc ? l : r;                     // arrive at this node from the complete child
-        child_box(aabbs, keys, node_aabb, cur, b);
-    }
-    for (int guard = 0; node >= 0 && guard < 96; ++guard) {
-        // every box this thread wrote has completed before the ticket is taken
-        __builtin_amdgcn_s_waitcnt(0);
-        const uint32_t t = __hip_atomic_fetch_add(ticket + node, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (t == 0u) return;                  // the sibling's thread finishes this node
-        const int32_t nl = left[node], nr = right[node];
-        const bool mine_left = (nl == cur);
-        const int32_t sib = mine_left ? nr : nl;
-        // a leaf's box from the input; a node's, written by the first kernel
-        // or by a climb, with agent-scope loads (current for both)
-        float o[6];
-        if (sib >= 0) child_box(aabbs, keys, node_aabb, sib, o);
-        else load_box(node_aabb + (size_t)(-sib) * 6u, o);
-        float u[6];
-        unite(b, o, mine_left, u);
-#pragma unroll
-        for (int q = 0; q < 6; ++q) b[q] = u[q];
-        store_box(node_aabb + (size_t)node * 6u, b);
-        if (node == 0) return;
-        cur = -node;
-        node = parent[node];
-    }
+    __syncthreads();
+    for (uint32_t q = t; q < m; q += kThreads)
+        climb<false>(T, nullptr, &I, out, m, q, T.box[q * 3u], T.box[q * 3u + 1u], T.box[q * 3u + 2u]);
+    leave_roots(T, &I, 0u, m, roots + (size_t)blockIdx.x * kMaxRoots, nroots + blockIdx.x);
 }
 
 // The tree in depth-first order with skip indices, for walks without a
@@ -669,15 +821,57 @@ __global__ void __launch_bounds__(256) k_flatten(const unsigned long long* __res
 } // namespace bvhk
 
 // ---- host API ----
+namespace {
+
+using namespace bvhk;
+
+uint32_t ceil_div(uint32_t a, uint32_t b) { return a / b + (a % b ? 1u : 0u); }
+
+// A build's scratch for up to n leaves, in 8-byte words of one array: the
+// other key buffer of the sort, its histogram rows and status words, and the
+// open subtrees of the tree's levels.
+struct Scratch {
+    u64* keys = nullptr;
+    u64* status = nullptr;
+    Root* roots[2] = {nullptr, nullptr};     // written by even / odd levels
+    uint32_t *rows = nullptr, *totals = nullptr, *tickets = nullptr, *nroots[2] = {nullptr, nullptr};
+};
+constexpr size_t hist_rows(size_t n) {
+    const size_t b = (n + kThreads - 1u) / kThreads;
+    return b < kHistBlocks ? b : kHistBlocks;
+}
+constexpr size_t scratch_words(size_t n) {
+    const size_t tiles = (n + kTile - 1u) / kTile, wgs = (n + kTreeTile - 1u) / kTreeTile;
+    const size_t up = (wgs + kTreeGroup - 1u) / kTreeGroup;
+    return n + 2u + kPasses * kDigits * tiles + hist_rows(n) * (kThreads / 2u) + kThreads / 2u + 8u +
+           (wgs + up) * (kMaxRoots * sizeof(Root) / 8u) + wgs / 2u + up / 2u + 8u;
+}
+Scratch scratch_at(void* base, size_t n) {
+    const size_t tiles = (n + kTile - 1u) / kTile, wgs = (n + kTreeTile - 1u) / kTreeTile;
+    const size_t up = (wgs + kTreeGroup - 1u) / kTreeGroup;
+    Scratch c;
+    u64* p = static_cast<u64*>(base);
+    c.roots[0] = reinterpret_cast<Root*>(p); p += wgs * (kMaxRoots * sizeof(Root) / 8u);
+    c.roots[1] = reinterpret_cast<Root*>(p); p += up * (kMaxRoots * sizeof(Root) / 8u);
+    c.keys = p; p += n + 2u;
+    c.status = p; p += kPasses * kDigits * tiles;
+    c.rows = reinterpret_cast<uint32_t*>(p); p += hist_rows(n) * (kThreads / 2u);
+    c.totals = reinterpret_cast<uint32_t*>(p); p += kThreads / 2u;
+    c.tickets = reinterpret_cast<uint32_t*>(p); p += 8u;
+    c.nroots[0] = reinterpret_cast<uint32_t*>(p); p += wgs / 2u + 4u;
+    c.nroots[1] = reinterpret_cast<uint32_t*>(p);
+    return c;
+}
+
+} // namespace
+
 struct pga_lbvh {
     uint32_t capacity = 0;
     int device = 0;
     hipStream_t stream = nullptr;
-    uint32_t *code[2] = {nullptr, nullptr}, *idx[2] = {nullptr, nullptr};
-    uint32_t* hist = nullptr;       // 256 x sort workgroups
-    uint32_t* part = nullptr;       // scan partials
-    uint32_t* ticket = nullptr;     // internal nodes
-    int32_t* other_end = nullptr;   // internal nodes: the far end of each node's leaf range
+    void* scratch_mem = nullptr;
+    Scratch scratch;
+    int32_t* other_end = nullptr;   // counted builds (pga_lbvh_enqueue_counted): see TreeOut
     float* bounds = nullptr;        // bounds partials; [0, 6) the folded scene box
     uint32_t* dev_words = nullptr;  // [0] leaf count of the last gather, [1] its overflow flag
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -685,8 +879,6 @@ struct pga_lbvh {
 };
 
 namespace {
-
-using namespace bvhk;
 
 pga_status lfail(pga_lbvh* b, pga_status st, const std::string& m) {
     if (b) b->error = m;
@@ -699,58 +891,53 @@ pga_status lfail(pga_lbvh* b, pga_status st, const std::string& m) {
         if (e_ != hipSuccess) return lfail(b, PGA_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-uint32_t sort_blocks(uint32_t n) { return (n + kTile - 1u) / kTile; }
-
-// Morton codes to refit for n leaves (nd: the device count, n its bound),
-// with a host scene box (mn, ex) or the device box `box`.
-hipError_t enqueue_build(pga_lbvh* b, const float* aabbs, uint32_t n, const uint32_t* nd, const float mn[3],
-                         const float ex[3], const float* box, uint64_t* keys, int32_t* left, int32_t* right,
-                         int32_t* parent, int32_t* leaf_parent, float* node_aabb) {
-    hipStream_t s = b->stream;
-    const uint32_t g = (n + 255u) / 256u;
-    hipLaunchKernelGGL(k_morton, dim3(g), dim3(256), 0, s, aabbs, n, nd, mn[0], mn[1], mn[2], ex[0], ex[1], ex[2],
-                       box, b->code[0], b->idx[0]);
-    const uint32_t nb = sort_blocks(n);
-    const uint32_t nh = 256u * nb;
-    const uint32_t np = (nh + kScanTile - 1u) / kScanTile;
-    int cur = 0;
-    for (uint32_t pass = 0; pass < 4; ++pass) {     // 30-bit codes: digits at bits 0, 8, 16, 24
-        const uint32_t shift = 8u * pass;
-        hipLaunchKernelGGL(k_hist, dim3(nb), dim3(kThreads), 0, s, b->code[cur], n, nd, shift, b->hist, nb);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(np), dim3(kThreads), 0, s, b->hist, nh, b->part);
-        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kThreads), 0, s, b->part, np);
-        hipLaunchKernelGGL(k_scan_down, dim3(np), dim3(kThreads), 0, s, b->hist, nh, b->part);
-        unsigned long long* keys_out = pass == 3 ? reinterpret_cast<unsigned long long*>(keys) : nullptr;
-        hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(kThreads), 0, s, b->code[cur], b->idx[cur], b->code[cur ^ 1],
-                           b->idx[cur ^ 1], keys_out, n, nd, shift, b->hist, nb);
-        cur ^= 1;
+// Morton keys, sort and tree for n leaves (nd: the device count, n its
+// bound), with a host scene box (mn, ex) or the device box `box`. other_end:
+// see TreeOut.
+hipError_t enqueue_build(const Scratch& c, hipStream_t s, const float* aabbs, uint32_t n, const uint32_t* nd,
+                         const float mn[3], const float ex[3], const float* box, uint64_t* keys_out, int32_t* left,
+                         int32_t* right, int32_t* parent, int32_t* leaf_parent, float* node_aabb,
+                         int32_t* other_end) {
+    const Scene scene{mn[0], mn[1], mn[2], ex[0], ex[1], ex[2], box};
+    u64* keys = reinterpret_cast<u64*>(keys_out);
+    if (n <= kSmallLeaves) {
+        hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kThreads), 0, s, aabbs, n, nd, scene, keys);
+    } else {
+        const uint32_t nb = ceil_div(n, kTile), rows = (uint32_t)hist_rows(n);
+        hipLaunchKernelGGL(k_morton, dim3(rows), dim3(kThreads), 0, s, aabbs, n, nd, scene, keys, c.rows, c.status,
+                           kPasses * kDigits * nb, c.tickets);
+        hipLaunchKernelGGL(k_digit_totals, dim3(kPasses * kDigits / 64u), dim3(kThreads), 0, s, c.rows, rows,
+                           c.totals);
+        for (uint32_t pass = 0; pass < kPasses; ++pass)     // an even number of passes: the last one writes `keys`
+            hipLaunchKernelGGL(k_sweep, dim3(nb), dim3(kThreads), 0, s, pass & 1u ? c.keys : keys,
+                               pass & 1u ? keys : c.keys, n, nd, pass, c.totals,
+                               c.status + (size_t)pass * kDigits * nb, c.tickets);
     }
-    const unsigned long long* k64 = reinterpret_cast<const unsigned long long*>(keys);
-    hipLaunchKernelGGL(k_karras, dim3(g), dim3(256), 0, s, k64, n, nd, left, right, parent, leaf_parent,
-                       b->other_end, b->ticket);
-    hipLaunchKernelGGL(k_refit_local, dim3((n + kRefitTile - 1u) / kRefitTile), dim3(256), 0, s, aabbs, k64, n, nd,
-                       left, right, parent, leaf_parent, b->other_end, node_aabb);
-    hipLaunchKernelGGL(k_refit_global, dim3(g), dim3(256), 0, s, aabbs, k64, n, nd, left, right, parent,
-                       b->other_end, node_aabb, b->ticket);
+    const TreeOut out{left, right, parent, leaf_parent, other_end, node_aabb};
+    uint32_t groups = ceil_div(n, kTreeTile), level = 0;
+    hipLaunchKernelGGL(k_tree_leaves, dim3(groups), dim3(kThreads), 0, s, aabbs, keys, n, nd, out, c.roots[0],
+                       c.nroots[0]);
+    while (groups > 1u) {
+        const uint32_t next = ceil_div(groups, kTreeGroup), from = level & 1u;
+        hipLaunchKernelGGL(k_tree_roots, dim3(next), dim3(kThreads), 0, s, keys, n, nd, out, c.roots[from],
+                           c.nroots[from], groups, c.roots[from ^ 1u], c.nroots[from ^ 1u]);
+        groups = next;
+        ++level;
+    }
     return hipGetLastError();
 }
 
 // ---- the allocation-free build (pga_lbvh_build_noalloc) ----
-// Its sort and refit scratch is this file-scope device array: two code and
-// two index arrays, the tickets and range ends of the internal nodes (4 bytes
-// per leaf each), the digit histograms and the scan partials, for at most
-// kNoAllocLeaves leaves (about 24.3 MiB, held by every GPU the library runs
-// on until the process ends). Host code uses the address that
-// hipGetSymbolAddress gives on each device, never the array's name.
+// Its scratch is this file-scope device array, for at most kNoAllocLeaves
+// leaves (about 16.1 MiB, held by every GPU the library runs on until the
+// process ends). Host code uses the address that hipGetSymbolAddress gives on
+// each device, never the array's name.
 constexpr uint32_t kNoAllocLeaves = PGA_LBVH_NOALLOC_MAX_LEAVES;
-constexpr size_t kNoAllocHist = (size_t)256 * ((kNoAllocLeaves + kTile - 1u) / kTile);
-constexpr size_t kNoAllocPart = (kNoAllocHist + kScanTile - 1u) / kScanTile + 1u;
-constexpr size_t kNoAllocWords = 6u * (size_t)kNoAllocLeaves + kNoAllocHist + kNoAllocPart;
-static __device__ __align__(256) uint32_t scratch[kNoAllocWords];
+static __device__ __align__(256) u64 scratch[scratch_words(kNoAllocLeaves)];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
-uint32_t* g_scratch[kMaxDevices] = {nullptr};   // the array's address on each device
+void* g_scratch[kMaxDevices] = {nullptr};   // the array's address on each device
 thread_local std::string g_noalloc_error;      // message of the last failed call on this thread
 
 pga_status noalloc_fail(pga_status st, const std::string& m) {
@@ -759,7 +946,7 @@ pga_status noalloc_fail(pga_status st, const std::string& m) {
 }
 
 // The array's address on the current device, looked up once per device.
-pga_status scratch_on_device(uint32_t** out) {
+pga_status scratch_on_device(void** out) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return noalloc_fail(PGA_ERR_HIP, std::string("hipGetDevice: ") + hipGetErrorString(e));
@@ -770,7 +957,7 @@ pga_status scratch_on_device(uint32_t** out) {
         e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p)
             return noalloc_fail(PGA_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        g_scratch[dev] = static_cast<uint32_t*>(p);
+        g_scratch[dev] = p;
     }
     *out = g_scratch[dev];
     return PGA_OK;
@@ -791,24 +978,12 @@ PGA_API pga_status pga_lbvh_build_noalloc(const float* aabbs, uint32_t n, const 
                                                      std::to_string(n));
     const float ex[3] = {scene_max[0] - scene_min[0], scene_max[1] - scene_min[1], scene_max[2] - scene_min[2]};
     if (!(ex[0] > 0.0f) || !(ex[1] > 0.0f) || !(ex[2] > 0.0f)) return noalloc_fail(PGA_ERR_INVALID_ARG, "empty scene box");
-    uint32_t* base = nullptr;
+    void* base = nullptr;
     pga_status st = scratch_on_device(&base);
     if (st) return st;
-    // a builder view of the array, sized for n leaves (no events, no allocation)
-    pga_lbvh view;
-    view.capacity = n;
-    view.stream = (hipStream_t)stream;
-    const size_t N = kNoAllocLeaves;
-    view.code[0] = base;
-    view.code[1] = base + N;
-    view.idx[0] = base + 2u * N;
-    view.idx[1] = base + 3u * N;
-    view.ticket = base + 4u * N;
-    view.other_end = reinterpret_cast<int32_t*>(base + 5u * N);
-    view.hist = base + 6u * N;
-    view.part = base + 6u * N + kNoAllocHist;
-    const hipError_t e = enqueue_build(&view, aabbs, n, nullptr, scene_min, ex, nullptr, keys, left, right, parent,
-                                       leaf_parent, node_aabb);
+    const hipError_t e = enqueue_build(scratch_at(base, kNoAllocLeaves), (hipStream_t)stream, aabbs, n, nullptr,
+                                       scene_min, ex, nullptr, keys, left, right, parent, leaf_parent, node_aabb,
+                                       nullptr);
     if (e != hipSuccess) return noalloc_fail(PGA_ERR_HIP, std::string("launch: ") + hipGetErrorString(e));
     return PGA_OK;
 }
@@ -821,14 +996,8 @@ PGA_API pga_status pga_lbvh_create(uint32_t capacity, int32_t device, void* stre
     if (device >= 0) LHIP(b, hipSetDevice(device));
     LHIP(b, hipGetDevice(&b->device));
     b->stream = (hipStream_t)stream;
-    for (int k = 0; k < 2; ++k) {
-        LHIP(b, hipMalloc((void**)&b->code[k], (size_t)capacity * 4u));
-        LHIP(b, hipMalloc((void**)&b->idx[k], (size_t)capacity * 4u));
-    }
-    const size_t nh = (size_t)256 * sort_blocks(capacity);
-    LHIP(b, hipMalloc((void**)&b->hist, nh * 4u));
-    LHIP(b, hipMalloc((void**)&b->part, ((nh + kScanTile - 1) / kScanTile + 1) * 4u));
-    LHIP(b, hipMalloc((void**)&b->ticket, (size_t)capacity * 4u));
+    LHIP(b, hipMalloc(&b->scratch_mem, scratch_words(capacity) * 8u));
+    b->scratch = scratch_at(b->scratch_mem, capacity);
     LHIP(b, hipMalloc((void**)&b->other_end, (size_t)capacity * 4u));
     LHIP(b, hipMalloc((void**)&b->bounds, 1024u * 6u * 4u));
     LHIP(b, hipMalloc((void**)&b->dev_words, 64u));
@@ -842,8 +1011,7 @@ PGA_API void pga_lbvh_destroy(pga_lbvh* b) {
     if (!b) return;
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     else (void)hipDeviceSynchronize();
-    for (int k = 0; k < 2; ++k) { (void)hipFree(b->code[k]); (void)hipFree(b->idx[k]); }
-    (void)hipFree(b->hist); (void)hipFree(b->part); (void)hipFree(b->ticket); (void)hipFree(b->bounds);
+    (void)hipFree(b->scratch_mem); (void)hipFree(b->bounds);
     (void)hipFree(b->dev_words); (void)hipFree(b->other_end);
     if (b->e0) (void)hipEventDestroy(b->e0);
     if (b->e1) (void)hipEventDestroy(b->e1);
@@ -883,8 +1051,8 @@ PGA_API pga_status pga_lbvh_build(pga_lbvh* b, const float* aabbs, uint32_t n, c
     const float ex[3] = {scene_max[0] - scene_min[0], scene_max[1] - scene_min[1], scene_max[2] - scene_min[2]};
     if (!(ex[0] > 0.0f) || !(ex[1] > 0.0f) || !(ex[2] > 0.0f)) return lfail(b, PGA_ERR_INVALID_ARG, "empty scene box");
     LHIP(b, hipEventRecord(b->e0, b->stream));
-    LHIP(b, enqueue_build(b, aabbs, n, nullptr, scene_min, ex, nullptr, keys, left, right, parent, leaf_parent,
-                          node_aabb));
+    LHIP(b, enqueue_build(b->scratch, b->stream, aabbs, n, nullptr, scene_min, ex, nullptr, keys, left, right, parent,
+                          leaf_parent, node_aabb, nullptr));
     LHIP(b, hipEventRecord(b->e1, b->stream));
     LHIP(b, hipStreamSynchronize(b->stream));
     return PGA_OK;
@@ -928,15 +1096,15 @@ PGA_API pga_status pga_lbvh_build_device(pga_lbvh* b, const float* aabbs, const 
         const float ex[3] = {scene_max[0] - scene_min[0], scene_max[1] - scene_min[1], scene_max[2] - scene_min[2]};
         if (!(ex[0] > 0.0f) || !(ex[1] > 0.0f) || !(ex[2] > 0.0f))
             return lfail(b, PGA_ERR_INVALID_ARG, "empty scene box");
-        LHIP(b, enqueue_build(b, aabbs, n, nd, scene_min, ex, nullptr, keys, left, right, parent, leaf_parent,
-                              node_aabb));
+        LHIP(b, enqueue_build(b->scratch, b->stream, aabbs, n, nd, scene_min, ex, nullptr, keys, left, right, parent,
+                              leaf_parent, node_aabb, nullptr));
     } else {
         const uint32_t blocks = std::min<uint32_t>(1024u, (n + 255u) / 256u);
         hipLaunchKernelGGL(k_bounds, dim3(blocks), dim3(256), 0, b->stream, aabbs, n, nd, b->bounds);
         hipLaunchKernelGGL(k_bounds_fold, dim3(1), dim3(256), 0, b->stream, b->bounds, blocks);
         const float zero[3] = {0.0f, 0.0f, 0.0f}, one[3] = {1.0f, 1.0f, 1.0f};
-        LHIP(b, enqueue_build(b, aabbs, n, nd, zero, one, b->bounds, keys, left, right, parent, leaf_parent,
-                              node_aabb));
+        LHIP(b, enqueue_build(b->scratch, b->stream, aabbs, n, nd, zero, one, b->bounds, keys, left, right, parent,
+                              leaf_parent, node_aabb, nullptr));
     }
     if (timed) LHIP(b, hipEventRecord(b->e1, b->stream));
     return PGA_OK;
@@ -955,8 +1123,8 @@ hipError_t pga_lbvh_enqueue_counted(pga_lbvh* b, const float* aabbs, const uint3
     hipLaunchKernelGGL(k_bounds, dim3(blocks), dim3(256), 0, b->stream, aabbs, n, nd, b->bounds);
     hipLaunchKernelGGL(k_bounds_fold, dim3(1), dim3(256), 0, b->stream, b->bounds, blocks);
     const float zero[3] = {0.0f, 0.0f, 0.0f}, one[3] = {1.0f, 1.0f, 1.0f};
-    const hipError_t e = enqueue_build(b, aabbs, n, nd, zero, one, b->bounds, keys, left, right, parent,
-                                       leaf_parent, node_aabb);
+    const hipError_t e = enqueue_build(b->scratch, b->stream, aabbs, n, nd, zero, one, b->bounds, keys, left, right,
+                                       parent, leaf_parent, node_aabb, b->other_end);
     if (e != hipSuccess) return e;
     const uint32_t g = (uint32_t)(((uint64_t)2u * n + 255u) / 256u);
     hipLaunchKernelGGL(k_flatten, dim3(g), dim3(256), 0, b->stream, reinterpret_cast<const unsigned long long*>(keys),

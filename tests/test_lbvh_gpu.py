@@ -56,6 +56,27 @@ def test_lbvh_matches_oracle(n, clustered):
     _compare(got, ref, n)
 
 
+def _skewed(n, seed):
+    """Centres at 2^-k of the scene from its corner: a deep, lopsided tree
+    with many open subtrees at every tile's edge."""
+    rng = np.random.default_rng(seed)
+    c = f32(100.0) * np.exp2(-rng.integers(0, 11, size=(n, 3))).astype(f32)
+    return np.concatenate([c - f32(0.001), c + f32(0.001)], axis=1).astype(f32)
+
+
+# one workgroup's sort and one tile of the tree, a leaf more than each, the
+# edges of the sort's tiles, one more tile than a group of the tree's second
+# level takes, and a third level
+@pytest.mark.parametrize("boxes", [_boxes, _skewed, lambda n, seed: np.tile(_boxes(1, seed), (n, 1))],
+                         ids=["spread", "skewed", "equal"])
+@pytest.mark.parametrize("n", [2, 63, 1023, 1024, 1025, 4095, 4096, 4097, 8192, 8193, 32769, 65537])
+def test_lbvh_tile_edges(n, boxes):
+    _note(f"lbvh tile edges n={n}")
+    b = boxes(n, n)
+    smin, smax = (0.0, 0.0, 0.0), (101.0, 101.0, 101.0)
+    _compare(_gpu_build(b, smin, smax), O.lbvh(b, smin, smax), n)
+
+
 def _np_instance_boxes(inst, planar):
     m = inst["model"].astype(f32)
     h = [np.abs(m[:, 4 * r]) + np.abs(m[:, 4 * r + 1]) for r in range(3)]
