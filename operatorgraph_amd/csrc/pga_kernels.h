@@ -16,6 +16,10 @@ constexpr uint32_t kBarWords = 192;     // grid barrier: generation + 9 counters
 // hand out and the parents / descriptors spilled from workgroup-local
 // frontiers to the grid's arrays
 constexpr uint32_t kBarGrab = 160, kBarSpillPar = 161, kBarSpillDesc = 162;
+// and what block 0 hands to the other blocks after the narrow levels it ran
+// alone: the next level, its children, and the tape's record and descriptor
+// bases of the previous / the next level
+constexpr uint32_t kBarLevel = 163, kBarChildren = 164, kBarTape = 165;
 
 struct KArgs {
     Prog prog;                          // tables in the global program image

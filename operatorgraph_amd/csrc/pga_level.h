@@ -22,6 +22,7 @@ struct LevelLDS {
     uint32_t next_n;                   // children of the next level (all blocks agree)
     uint32_t grab;                     // workgroup-local derivation: first axiom handed to this block
     uint32_t spill;                    // ... 1: this level's fan-outs go to the grid's arrays
+    uint32_t gen;                      // grid_barrier: barriers since the reset (thread 0's)
     uint32_t tp_prev, tp_cur;          // tape: parent-record base of the previous / this level
     uint32_t td_prev, td_cur;          // tape: descriptor base of the previous / this level
 };
@@ -46,9 +47,13 @@ __device__ __forceinline__ void store_rec(Rec* dst, const Rec& r) {
     d[3] = make_float4(r.s[0], r.s[1], r.s[2], r.seed);
     d[4] = make_float4(r.custom, __uint_as_float(r.ed), __uint_as_float(r.axiom), __uint_as_float(r.path));
 }
-__device__ __forceinline__ void load_rec(const Rec* src, Rec& r) {
+// geom false: nothing reads the model (a count pass), 48 of the 80 bytes stay
+// where they are.
+__device__ __forceinline__ void load_rec(const Rec* src, Rec& r, bool geom = true) {
     const float4* s = reinterpret_cast<const float4*>(src);
-    float4 a = s[0], b = s[1], c = s[2], d = s[3], e = s[4];
+    float4 a = {}, b = {}, c = {};
+    if (geom) { a = s[0]; b = s[1]; c = s[2]; }
+    const float4 d = s[3], e = s[4];
     r.m[0] = a.x; r.m[1] = a.y; r.m[2] = a.z; r.m[3] = a.w;
     r.m[4] = b.x; r.m[5] = b.y; r.m[6] = b.z; r.m[7] = b.w;
     r.m[8] = c.x; r.m[9] = c.y; r.m[10] = c.z; r.m[11] = c.w;
@@ -361,19 +366,25 @@ __device__ __forceinline__ bool load_axiom(const KArgs& a, const Ctx& c, uint32_
     return true;
 }
 
+// The descriptor of child i (level 0 has none). The passes read it an
+// iteration ahead: the parent it names is one more dependent load, and at two
+// or three waves per SIMD the two round trips were most of a count pass.
+__device__ __forceinline__ uint4 load_desc(const Desc* desc_in, uint32_t level, uint32_t i, uint32_t n) {
+    return level != 0u && i < n ? *reinterpret_cast<const uint4*>(desc_in + i) : make_uint4(0u, kDescNone, 0u, 0u);
+}
+
 template <class Visit>
 __device__ __forceinline__ bool load_child_at(const KArgs& a, const Ctx& c, uint32_t first, const Rec* par_in,
-                                              uint32_t in_cap, const Desc* desc_in, bool wr, uint32_t level,
+                                              uint32_t in_cap, uint4 dv, bool wr, uint32_t level,
                                               uint32_t i, Rec& r, Visit visit) {
     if (level == 0u) return load_axiom(a, c, first + i, wr, r);
-    const uint4 dv = *reinterpret_cast<const uint4*>(desc_in + i);
     const uint32_t parent = dv.x, jx = dv.y;
     const uint32_t j = jx & 0x3FFFFFFFu;
     if (j == kDescAxiom) return load_axiom(a, c, parent, wr, r);
     if (parent >= in_cap) return false;          // parent was dropped on overflow
     if (j == kDescNone) return false;
     Rec p;
-    load_rec(par_in + parent, p);
+    load_rec(par_in + parent, p, c.geom != 0u);
     if (j == kDescSelf) { r = p; return true; }
     bool ok = false;
     visit(c, rec_entry(p), [&](const auto& e) {
@@ -384,40 +395,44 @@ __device__ __forceinline__ bool load_child_at(const KArgs& a, const Ctx& c, uint
 
 // The same over the launch's axioms and the grid's parent arrays.
 template <class Visit = LoadEntry>
-__device__ __forceinline__ bool load_child(const KArgs& a, const Ctx& c, const Rec* par_in, const Desc* desc_in,
+__device__ __forceinline__ bool load_child(const KArgs& a, const Ctx& c, const Rec* par_in, uint4 dv,
                                            bool wr, uint32_t level, uint32_t i, Rec& r, Visit visit = Visit()) {
-    return load_child_at(a, c, a.first_axiom, par_in, a.cap_par, desc_in, wr, level, i, r, visit);
+    return load_child_at(a, c, a.first_axiom, par_in, a.cap_par, dv, wr, level, i, r, visit);
 }
 
 // Grid-wide barrier of a cooperative launch. Words (64 bytes apart):
 // bar[0] generation, bar[16 (g + 1)] arrivals of block group g = block % 8,
 // bar[16 * 9] arrivals of the groups. Spreading the arrivals over nine
-// counters keeps same-address atomics short; every counter is back at 0 and
-// the generation one higher after each barrier. One agent-scope release
-// fence per block before arriving, relaxed polling, one acquire fence after.
-__device__ __forceinline__ void grid_barrier(uint32_t* bar, uint32_t nblocks) {
+// counters keeps same-address atomics short. The counters only grow (the
+// n-th barrier since the reset ends at n times the arrivals), so none has to
+// be back at 0 before the next barrier, and `gen` (LDS, thread 0's) is the
+// block's copy of the generation. One agent-scope release fence per block
+// before arriving, relaxed polling, one acquire fence after.
+// FENCED = false: for data that crosses the barrier in agent-scope atomic
+// accesses only, whose writers have waited for them (scan_counts); the fences
+// write back and invalidate caches the next pass reads from.
+template <bool FENCED = true>
+__device__ __forceinline__ void grid_barrier(uint32_t* bar, uint32_t nblocks, uint32_t& gen) {
     __syncthreads();
     if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const uint32_t gen = __hip_atomic_load(&bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (FENCED) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const uint32_t next = gen + 1u;
         const uint32_t g = blockIdx.x & 7u;
         const uint32_t in_group = (nblocks - g + 7u) >> 3;          // blocks b < nblocks with b % 8 == g
         const uint32_t groups = nblocks < 8u ? nblocks : 8u;
-        bool last = false;
-        uint32_t* gc = &bar[16u * (g + 1u)];
-        if (__hip_atomic_fetch_add(gc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == in_group - 1u) {
-            __hip_atomic_store(gc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t* top = &bar[16u * 9u];
-            last = __hip_atomic_fetch_add(top, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1u;
-            if (last) __hip_atomic_store(top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        const bool last =
+            __hip_atomic_fetch_add(&bar[16u * (g + 1u)], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                next * in_group - 1u &&
+            __hip_atomic_fetch_add(&bar[16u * 9u], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                next * groups - 1u;
         if (last) {
-            __hip_atomic_store(&bar[0], gen + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&bar[0], next, FENCED ? __ATOMIC_RELEASE : __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-            while (__hip_atomic_load(&bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen)
+            while (__hip_atomic_load(&bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != next)
                 __builtin_amdgcn_s_sleep(1);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        gen = next;
+        if (FENCED) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
 }
@@ -444,14 +459,20 @@ __device__ __forceinline__ void scan_counts(const KArgs& a, LevelLDS& L, uint32_
             L.cur[ww][k] = s;
             s += L.cnt[ww][k];
         }
-        totals[k] = s;
+        __hip_atomic_store(&totals[k], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    grid_barrier(a.bar, gridDim.x);
+    // the totals are all that crosses this barrier: written and read at agent
+    // scope, complete before the block arrives. With the fences of
+    // grid_barrier a scan took 5.5 us at 256 workgroups, and the write pass
+    // read the children the count pass had just read from memory again
+    __builtin_amdgcn_s_waitcnt(0);
+    grid_barrier<false>(a.bar, gridDim.x, L.gen);
     // wave w sums counters k = w, w + nw, ... over the blocks, 64 blocks a step
     for (uint32_t k = wave_in_block(); k < ncnt; k += nw) {
         uint32_t before = 0, all = 0;
         for (uint32_t b = lane_id(); b < gridDim.x; b += 64u) {
-            const uint32_t v = a.block_totals[(size_t)b * ncnt + k];
+            const uint32_t v = __hip_atomic_load(&a.block_totals[(size_t)b * ncnt + k], __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
             all += v;
             before += b < blockIdx.x ? v : 0u;
         }
@@ -475,6 +496,35 @@ __device__ __forceinline__ void scan_counts(const KArgs& a, LevelLDS& L, uint32_
     }
     __syncthreads();
     stamp(a, row, 2);
+}
+
+// The scan of a level that one block runs alone: its waves' offsets and the
+// level's totals.
+__device__ __forceinline__ void scan_block(const KArgs& a, LevelLDS& L, uint32_t level) {
+    const uint32_t nslots = a.prog.nslots, ncnt = nslots + 2u;
+    stamp(a, level, 1);
+    const uint32_t nw = blockDim.x >> 6;
+    for (uint32_t k = threadIdx.x; k < ncnt; k += blockDim.x) {
+        uint32_t s = 0;
+        for (uint32_t ww = 0; ww < nw; ++ww) {
+            L.cur[ww][k] = s;
+            s += L.cnt[ww][k];
+        }
+        L.level_total[k] = s;
+        if (k == nslots) a.par_counts[level] = s;
+        if (k == nslots + 1u) {
+            a.desc_counts[level] = s;
+            L.next_n = s;
+        }
+    }
+    __syncthreads();
+    stamp(a, level, 2);
+}
+
+// The barriers passed before this launch (KERNELS: earlier levels).
+__device__ __forceinline__ void init_barrier(const KArgs& a, LevelLDS& L) {
+    if (threadIdx.x == 0)
+        L.gen = __hip_atomic_load(&a.bar[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void init_bases(const KArgs& a, LevelLDS& L) {

@@ -176,12 +176,14 @@ __device__ __forceinline__ void spec_pass(const KArgs& a, LevelLDS& L, float4* P
     c.desc_cap = io.desc_cap;
     const SpecVisit<S> visit;
     f4* ST = reinterpret_cast<f4*>(PW + 5u * blockDim.x) + wave_in_block() * 256u;
+    uint4 dnext = load_desc(io.desc_in, level, wave * 64u + lane_id(), n);
 #pragma unroll 1
     for (uint32_t base = wave * 64u; base < n; base += nwaves * 64u) {
         const uint32_t i = base + lane_id();
+        const uint4 dv = dnext;
+        dnext = load_desc(io.desc_in, level, i + nwaves * 64u, n);
         Rec cur;
-        const bool valid = i < n && load_child_at(a, c, io.first, io.par_in, io.in_cap, io.desc_in, WR, level, i,
-                                                  cur, visit);
+        const bool valid = i < n && load_child_at(a, c, io.first, io.par_in, io.in_cap, dv, WR, level, i, cur, visit);
         uint32_t mode = valid ? M_SETTLE : M_DONE;
         bool leaf = false, self = false;
         uint32_t steps = 0, j = 0, dslot = 0, pidx = ~0u, fe = 0;
@@ -421,6 +423,7 @@ __device__ __forceinline__ void spec_mega(const KArgs& a) {
     __shared__ LevelLDS L;
     __shared__ float4 PW[9 * BS];   // parent records (5 words per lane), then instance staging (4)
     stage_program(a);
+    init_barrier(a, L);
     const uint32_t nslots = a.prog.nslots, ncnt = nslots + 2u;
     const uint32_t w = wave_in_block();
     const uint32_t kp = a.loc_kp, kd = a.loc_kd;
@@ -457,7 +460,7 @@ __device__ __forceinline__ void spec_mega(const KArgs& a) {
                 __syncthreads();
             }
             if (n == 0u) {          // nothing held and nothing left: the grid-wide levels
-                grid_barrier(a.bar, gridDim.x);     // every spill and instance claim is done
+                grid_barrier(a.bar, gridDim.x, L.gen);     // every spill and instance claim is done
                 const uint32_t spilled =
                     __hip_atomic_load(&a.bar[kBarSpillDesc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (blockIdx.x == 0 && threadIdx.x == 0) a.desc_counts[0] = spilled;
@@ -525,7 +528,7 @@ __device__ __forceinline__ void spec_mega(const KArgs& a) {
                 for (uint32_t k = 0; k < nslots; ++k) L.term_base[k] += L.level_total[k];
             __syncthreads();
             n = min(L.next_n, a.cap_desc);
-            grid_barrier(a.bar, gridDim.x);       // next level reads this level's records
+            grid_barrier(a.bar, gridDim.x, L.gen);       // next level reads this level's records
         }
         ++level;
     }

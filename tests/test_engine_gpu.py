@@ -92,6 +92,20 @@ def test_stochastic_philox(E, technique):
     check_against_oracle(E, grammars.stochastic(), ax, 1, technique, key=axioms.STOCHASTIC_KEY)
 
 
+@pytest.mark.parametrize("block_size", [256, 512])
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 511, 512, 513, 1025])
+def test_narrow_and_wide_levels(E, n, block_size):
+    """Levels that one block runs alone (at most block_size children) and
+    grid-wide ones in one derivation: the stochastic batch widens, then
+    narrows down to nothing, from either side of both widths."""
+    _note(f"narrow and wide levels n={n} block_size={block_size}")
+    ax, _ = axioms.stochastic_axioms(n)
+    _, st = check_against_oracle(E, grammars.stochastic(), ax, 1, abi.MEGAKERNEL, key=axioms.STOCHASTIC_KEY,
+                                 twins=False, block_size=block_size)
+    _, ref = gpu_derive(E, grammars.stochastic(), ax, 1, abi.KERNELS, key=axioms.STOCHASTIC_KEY, block_size=block_size)
+    assert (st["levels"], st["records"], st["terminals"]) == (ref["levels"], ref["records"], ref["terminals"])
+
+
 @pytest.mark.parametrize("technique", TECHNIQUES)
 def test_param_facade(E, technique):
     _note(f"parametrised facade technique={technique}")
