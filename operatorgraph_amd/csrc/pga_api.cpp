@@ -1428,7 +1428,7 @@ PGA_API pga_status pga_specialize(pga_context* ctx, uint32_t block_size, int32_t
     }
     drop_spec(ctx);
     const auto t0 = std::chrono::steady_clock::now();
-    const std::string src = pga_spec_source(ctx->h_entries, ctx->count_geom, ctx->use_seed, block_size);
+    const std::string src = pga_spec_source(ctx->h_entries, ctx->h_params, ctx->h_succ, ctx->count_geom, ctx->use_seed, block_size);
     std::vector<char> code;
     std::string log;
     bool cached = false;
@@ -1481,7 +1481,7 @@ PGA_API pga_status pga_specialize_check(const pga_procedure* procedures, uint32_
         const auto t0 = std::chrono::steady_clock::now();
         std::vector<char> code;
         bool cached = false;
-        if (!pga_spec_compile(pga_spec_source(ctx->h_entries, ctx->count_geom, ctx->use_seed, block_size), code, msg,
+        if (!pga_spec_compile(pga_spec_source(ctx->h_entries, ctx->h_params, ctx->h_succ, ctx->count_geom, ctx->use_seed, block_size), code, msg,
                               &cached))
             st = PGA_ERR_UNSUPPORTED;
         else if (seconds && !cached)

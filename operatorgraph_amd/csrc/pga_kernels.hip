@@ -44,6 +44,7 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
     const Rec* par_in = TAPE ? a.tape_par + L.tp_prev : ((level & 1u) ? a.par0 : a.par1);
     const Desc* desc_in = TAPE ? a.tape_desc + L.td_prev : ((level & 1u) ? a.desc0 : a.desc1);
     const uint32_t child_base = level == 0u ? 0u : a.n_axioms + L.td_prev;   // tape outcomes
+    f4* ST = reinterpret_cast<f4*>(PW + 5u * blockDim.x) + wave_in_block() * 256u;
     uint4 dnext = load_desc(desc_in, level, wave * 64u + lane_id(), n);
 #pragma unroll 1
     for (uint32_t base = wave * 64u; base < n; base += nwaves * 64u) {
@@ -67,7 +68,7 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
         uint32_t steps = 0, j = 0, dslot = 0, pidx = ~0u;
         uint32_t skipm = 0, nd = 0;   // children that go to a Discard; descriptors to write
         Fan f;
-        f.n = 0; f.axis = 0; f.total = 0.0f; f.r2a = 0.0f; f.off = 0.0f;
+        f.n = 0; f.axis = 0; f.total = 0.0f; f.r2a = 0.0f; f.off = 0.0f; f.c1 = 0.0f;
         f.e1 = f.e2 = f.e3 = 0.0f; f.prev_ns = 0.0f; f.prev_o = 0.0f; f.reps = 0;
 #pragma unroll 1
         while (__ballot(mode != M_DONE) != 0ull) {
@@ -170,8 +171,7 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
             }
             if (__ballot(emit) != 0ull) {
                 unsigned long long idx;
-                emit_terminal(c, L, reinterpret_cast<f4*>(PW + 5u * blockDim.x) + wave_in_block() * 256u, wr, emit, slot,
-                              cur, idx);
+                emit_terminal(c, L, ST, wr, emit, slot, cur, idx);
                 if (TAPE && emit) { out_kind = T_TERM | (slot << 8); out_a = (uint32_t)idx; }
             }
             if (__ballot(start) != 0ull) {

@@ -85,7 +85,10 @@ __device__ __forceinline__ uint32_t claim(LevelLDS& L, bool wr, uint32_t k, unsi
 // them out as consecutive 16-byte nontemporal stores: a lane storing its own
 // record would leave every store instruction a 64-byte stride, and partly
 // written lines cost more than the coalesced stream (measured 0.91 -> 0.80 ms
-// on 16,384 facade lots). The copy reads its (at most four) words per lane
+// on 16,384 facade lots). The four words of record r are rotated by r / 4
+// (stage_at), so that 16 lanes of either side of the copy touch 16 different
+// 16-byte columns of LDS: in place, the lanes writing word k of 16 records
+// met on four of them (41M conflict cycles on 16,384 lots). The copy reads its (at most four) words per lane
 // from LDS before any store, and stores through a global-memory pointer: a
 // flat store would also count against the LDS wait of the next read.
 // The instance record of a terminal shape as four 16-byte rows: model4 *
@@ -116,6 +119,38 @@ __device__ __forceinline__ void instance_rows(const Rec& r, bool inv, f4& q0, f4
     q3 = f4{r.custom, __uint_as_float(r.axiom), __uint_as_float(r.path), __uint_as_float(r.ed & ~kInvert)};
 }
 
+__device__ __forceinline__ uint32_t stage_at(uint32_t r, uint32_t k) { return r * 4u + ((k + (r >> 2)) & 3u); }
+
+// Stages the records of the lanes in `mask` (rank: the lane's among them) and
+// writes them out from dst on; records at or past `room` stay out.
+__device__ __forceinline__ void copy_out(f4* ST, gf4* dst, unsigned long long room, bool mine, uint32_t rank,
+                                         unsigned long long mask, f4 q0, f4 q1, f4 q2, f4 q3) {
+    if (mine) {
+        ST[stage_at(rank, 0u)] = q0;
+        ST[stage_at(rank, 1u)] = q1;
+        ST[stage_at(rank, 2u)] = q2;
+        ST[stage_at(rank, 3u)] = q3;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t n4 = (uint32_t)__popcll(mask) * 4u;
+    f4 v[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; ++u) {
+        const uint32_t q = lane_id() + 64u * u;
+        v[u] = q < n4 ? ST[stage_at(q >> 2, q & 3u)] : f4{};
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; ++u) {
+        const uint32_t q = lane_id() + 64u * u;
+        if (q < n4 && (q >> 2) < room) __builtin_nontemporal_store(v[u], dst + q);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ void emit_terminal(const Ctx& c, LevelLDS& L, f4* ST, bool wr, bool has, uint32_t slot,
                                               const Rec& r, unsigned long long& idx) {
     f4 q0 = {}, q1 = {}, q2 = {}, q3 = {};
@@ -134,58 +169,117 @@ __device__ __forceinline__ void emit_terminal(const Ctx& c, LevelLDS& L, f4* ST,
         const unsigned long long first = L.term_base[sl] + base;
         if (mine) idx = first + rank;
         if (wr) {
-            // the group's records are consecutive: stage them in rank order
-            // and write them out as consecutive 16-byte stores
-            if (mine) {
-                ST[rank * 4u + 0u] = q0;
-                ST[rank * 4u + 1u] = q1;
-                ST[rank * 4u + 2u] = q2;
-                ST[rank * 4u + 3u] = q3;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // the group's records are consecutive: staged in rank order and
+            // written out as consecutive 16-byte stores
             const uint32_t t = c.prog.slot_term[sl];
             const unsigned long long cap = c.inst_cap[t];
-            const uint32_t n4 = (uint32_t)__popcll(m) * 4u;
-            gf4* dst = (gf4*)(c.inst[t] + first);
-            f4 v[4];
-#pragma unroll
-            for (uint32_t u = 0; u < 4u; ++u) {
-                const uint32_t q = lane_id() + 64u * u;
-                v[u] = q < n4 ? ST[q] : f4{};
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < 4u; ++u) {
-                const uint32_t q = lane_id() + 64u * u;
-                if (q < n4 && first + (q >> 2) < cap) __builtin_nontemporal_store(v[u], dst + q);
-            }
+            copy_out(ST, (gf4*)(c.inst[t] + first), cap > first ? cap - first : 0ull, mine, rank, m, q0, q1, q2, q3);
             if (mine && idx >= cap && cap != 0ull) raise(c, PGA_ERR_OVERFLOW_INSTANCES);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
         pending &= ~m;
     }
 }
 
+// The record of each lane's current fan-out parent lives in LDS (five
+// 16-byte words per lane, word k of all lanes contiguous), not in registers:
+// the state machine then fits more waves per SIMD.
+__device__ __forceinline__ void par_store(float4* PW, const Rec& r) {
+    float4* p = PW + threadIdx.x;
+    const uint32_t s = blockDim.x;
+    p[0] = make_float4(r.m[0], r.m[1], r.m[2], r.m[3]);
+    p[s] = make_float4(r.m[4], r.m[5], r.m[6], r.m[7]);
+    p[2u * s] = make_float4(r.m[8], r.m[9], r.m[10], r.m[11]);
+    p[3u * s] = make_float4(r.s[0], r.s[1], r.s[2], r.seed);
+    p[4u * s] = make_float4(r.custom, __uint_as_float(r.ed), __uint_as_float(r.axiom), __uint_as_float(r.path));
+}
+__device__ __forceinline__ Rec par_load(const float4* PW) {
+    const float4* p = PW + threadIdx.x;
+    const uint32_t s = blockDim.x;
+    const float4 a = p[0], b = p[s], c = p[2u * s], d = p[3u * s], e = p[4u * s];
+    Rec r;
+    r.m[0] = a.x; r.m[1] = a.y; r.m[2] = a.z; r.m[3] = a.w;
+    r.m[4] = b.x; r.m[5] = b.y; r.m[6] = b.z; r.m[7] = b.w;
+    r.m[8] = c.x; r.m[9] = c.y; r.m[10] = c.z; r.m[11] = c.w;
+    r.s[0] = d.x; r.s[1] = d.y; r.s[2] = d.z; r.seed = d.w;
+    r.custom = e.x; r.ed = __float_as_uint(e.y); r.axiom = __float_as_uint(e.z); r.path = __float_as_uint(e.w);
+    return r;
+}
+
 // ---- direct leaf fan-outs in the write pass ----
 // A direct fan-out (EF_DIRECT: every child is a Generate of a constant
 // terminal, or a Discard) does not take each child round the state machine:
-// the wave's direct fan-outs emit their children in lock step, child j of
-// every such lane in round j (direct_child builds it), each round one
-// coalesced emit_terminal - the order in which the state machine would have
-// emitted them. The count pass takes the totals from the entry's table
-// (count_direct).
+// the lanes of the wave whose fan-out is entry e emit their children in lock
+// step, child j of every such lane in round j. The whole wave is here
+// (`mine`: the lane has such a fan-out, its parent record in PW): the parent
+// is read once, and so are the buffers and cursors of the entry's one or two
+// terminal slots. Where e is a type of constants the rounds are unrolled, and
+// a round is the child's arithmetic, its staging and its stores. The count
+// pass takes the totals from the entry's table (count_direct).
 template <class E>
-__device__ __forceinline__ bool direct_child(const Ctx& c, const Rec& par, const E& e, Fan& f, uint32_t skipm,
-                                             uint32_t j, Rec& ch, uint32_t& slot) {
-    float o = 0.0f, ns = 0.0f;
-    const bool keep = fan_geom(c, par, e, f, j, o, ns);
-    const bool skip = j < 32u ? ((skipm >> j) & 1u) != 0u : skipm == 0xFFFFFFFFu;
-    if (!keep || skip || !build_child(c, par, e, j, f.axis, o, ns, ch)) return false;
-    slot = c.prog.entries[rec_entry(ch)].tslot;
-    return true;
+constexpr uint32_t direct_rounds() {     // children of a constant entry's fan-out, 0: not a constant
+    if constexpr (E::kConst) {
+        return E::kind() == K_SUBDIV ? E::nparams() - 1u
+             : E::kind() == K_COMPSPLIT ? 6u : E::kind() == K_REPLICATE ? E::nsucc() : 0u;
+    }
+    return 0u;
+}
+template <class E>
+__device__ __forceinline__ void emit_direct(const Ctx& c, LevelLDS& L, f4* ST, const float4* PW, const E& e, bool mine,
+                                            Fan& f, uint32_t skipm) {
+    if (e.ndirect() == 0u) return;           // Discards only
+    const uint32_t w = wave_in_block(), tab = entry_aux(c, e, 1);
+    const Rec par = par_load(PW);
+    unsigned long long next[2], cap[2];
+    gf4* dst[2];
+#pragma unroll
+    for (uint32_t k = 0; k < 2u; ++k) {
+        const uint32_t slot = k < e.ndirect() ? (tab >> (16u * k)) & 0xFFu : (tab & 0xFFu);
+        const uint32_t t = c.prog.slot_term[slot];
+        next[k] = L.term_base[slot] + L.cur[w][slot];
+        cap[k] = c.inst_cap[t];
+        dst[k] = (gf4*)c.inst[t];
+    }
+    unsigned long long done[2] = {0ull, 0ull};
+    const uint32_t n = mine ? f.n : 0u;
+    const uint32_t kind = e.kind();
+    auto round = [&](uint32_t j) {
+        Rec ch;
+        bool has = false;
+        if (j < n) {
+            float o = 0.0f, ns = 0.0f;
+            const bool keep = fan_geom(c, par, e, f, j, o, ns);
+            const bool skip = j < 32u ? ((skipm >> j) & 1u) != 0u : skipm == 0xFFFFFFFFu;
+            has = keep && !skip && build_child(c, par, e, j, f.axis, o, ns, ch);
+        }
+        const unsigned long long m = __ballot(has);
+        if (m == 0ull) return;
+        // the child's slot: the successor's terminal, one of the table's
+        const uint32_t s = kind == K_REPEAT ? 0u : (kind == K_COMPSPLIT ? (j < 4u ? 2u : (j == 4u ? 1u : 0u)) : j);
+        const uint32_t slot = c.prog.entries[(uint32_t)succ_of(c, e, s) & 0x7FFFu].tslot;
+        const bool second = e.ndirect() > 1u && slot != (tab & 0xFFu);
+        const unsigned long long first = second ? next[1] + done[1] : next[0] + done[0];
+        const unsigned long long lim = second ? cap[1] : cap[0];
+        const uint32_t rank = mbcnt(m);
+        f4 q0 = {}, q1 = {}, q2 = {}, q3 = {};
+        if (has) instance_rows(ch, c.poly && (ch.ed & kInvert) != 0u, q0, q1, q2, q3);
+        copy_out(ST, (second ? dst[1] : dst[0]) + first * 4u, lim > first ? lim - first : 0ull, has, rank, m, q0, q1,
+                 q2, q3);
+        if (has && first + rank >= lim && lim != 0ull) raise(c, PGA_ERR_OVERFLOW_INSTANCES);
+        if (second) done[1] += (unsigned long long)__popcll(m);
+        else done[0] += (unsigned long long)__popcll(m);
+    };
+    constexpr uint32_t kRounds = direct_rounds<E>();
+    if constexpr (kRounds != 0u && kRounds <= 8u) {
+#pragma unroll
+        for (uint32_t j = 0; j < kRounds; ++j) round(j);
+    } else {
+#pragma unroll 1
+        for (uint32_t j = 0; __ballot(j < n) != 0ull; ++j) round(j);
+    }
+    if (lane_id() == 0) {
+        L.cur[w][tab & 0xFFu] += (uint32_t)done[0];
+        if (e.ndirect() > 1u) L.cur[w][(tab >> 16) & 0xFFu] += (uint32_t)done[1];
+    }
 }
 
 // Counting pass over a direct leaf fan-out: its children's terminals per
@@ -307,31 +401,6 @@ __device__ __forceinline__ Ctx make_ctx(const KArgs& a, const LevelLDS& L, uint3
     c.coll_bits = CS ? a.coll_bits : nullptr;
     c.coll_bits_cap = CS ? a.coll_bits_cap : 0u;
     return c;
-}
-
-// The record of each lane's current fan-out parent lives in LDS (five
-// 16-byte words per lane, word k of all lanes contiguous), not in registers:
-// the state machine then fits more waves per SIMD.
-__device__ __forceinline__ void par_store(float4* PW, const Rec& r) {
-    float4* p = PW + threadIdx.x;
-    const uint32_t s = blockDim.x;
-    p[0] = make_float4(r.m[0], r.m[1], r.m[2], r.m[3]);
-    p[s] = make_float4(r.m[4], r.m[5], r.m[6], r.m[7]);
-    p[2u * s] = make_float4(r.m[8], r.m[9], r.m[10], r.m[11]);
-    p[3u * s] = make_float4(r.s[0], r.s[1], r.s[2], r.seed);
-    p[4u * s] = make_float4(r.custom, __uint_as_float(r.ed), __uint_as_float(r.axiom), __uint_as_float(r.path));
-}
-__device__ __forceinline__ Rec par_load(const float4* PW) {
-    const float4* p = PW + threadIdx.x;
-    const uint32_t s = blockDim.x;
-    const float4 a = p[0], b = p[s], c = p[2u * s], d = p[3u * s], e = p[4u * s];
-    Rec r;
-    r.m[0] = a.x; r.m[1] = a.y; r.m[2] = a.z; r.m[3] = a.w;
-    r.m[4] = b.x; r.m[5] = b.y; r.m[6] = b.z; r.m[7] = b.w;
-    r.m[8] = c.x; r.m[9] = c.y; r.m[10] = c.z; r.m[11] = c.w;
-    r.s[0] = d.x; r.s[1] = d.y; r.s[2] = d.z; r.seed = d.w;
-    r.custom = e.x; r.ed = __float_as_uint(e.y); r.axiom = __float_as_uint(e.z); r.path = __float_as_uint(e.w);
-    return r;
 }
 
 // Calls f(entry) with entry i read from the program tables at run time (the

@@ -29,8 +29,11 @@ namespace pga {
 // fields are compile-time constants (kernels specialised to one program,
 // where the same operator code folds to the entry at hand). E provides the
 // fields idx, w0, w1, pbase, sbase, pv0..pv2, sv0, the accessors below, and
-// pvk / svk / auxk / param for fields chosen by index.
+// pvk / svk / auxk / param for fields chosen by index. kConst: all of them
+// are constants, also the parameters and successors beyond the third; loops
+// over them are then unrolled, so that every index is one.
 struct EntryV {
+    static constexpr bool kConst = false;
     uint32_t idx;     // entry index
     uint32_t w0;      // kind | shape << 8 | flags << 16 | nparams << 24
     uint32_t w1;      // nsucc | inl << 8 | tslot << 16 | ndirect << 24
@@ -51,7 +54,14 @@ struct EntryV {
     __device__ __forceinline__ uint32_t auxk(const Ctx& c, uint32_t k) const { return c.prog.entries[idx].aux[k]; }
     // parameter k (any k < nparams) from the program tables
     __device__ __forceinline__ DevParam param(const Ctx& c, uint32_t k) const { return c.prog.params[pbase + k]; }
+    // successor k >= 3
+    __device__ __forceinline__ int32_t svx(const Ctx& c, uint32_t k) const { return c.prog.succ[sbase + k]; }
+    // the axis of a Subdivide or Repeat, `a` unless it is a constant of the type
+    __device__ __forceinline__ uint32_t axis(uint32_t a) const { return a; }
 };
+// trips to unroll in loops over an entry's parameters or children
+template <class E>
+constexpr int kEntryUnroll = E::kConst ? 16 : 1;
 static_assert(sizeof(DevEntry) == 48, "DevEntry must be three 16-byte words");
 
 // Entry i of this lane, from the LDS copy of the program.
@@ -124,7 +134,7 @@ __device__ __forceinline__ float P(const Ctx& c, const E& e, uint32_t k, const R
 template <class E>
 __device__ __forceinline__ int32_t succ_of(const Ctx& c, const E& e, uint32_t k) {
     if (k < 3u) return e.svk(c, k);
-    return c.prog.succ[e.sbase + k];
+    return e.svx(c, k);
 }
 
 // The first min(nparams, 3) parameters; constants come from the entry, the
@@ -137,7 +147,7 @@ __device__ __forceinline__ void eval3(const Ctx& c, const E& e, const Rec& r, fl
     const uint32_t todo = ((1u << np) - 1u) & ~e.inl();
     if (todo == 0u) return;
     const uint32_t ax = r.axiom, pa = r.path, de = rec_depth(c, r);
-#pragma unroll 1
+#pragma unroll kEntryUnroll<E>
     for (uint32_t k = 0; k < np; ++k) {
         if (!((todo >> k) & 1u)) continue;
         float x = eval_param(c, e.param(c, k), r, ax, pa, de);
@@ -157,6 +167,7 @@ __device__ __forceinline__ int32_t random_choice(const Ctx& c, const E& e, float
     const uint32_t axiom = rr.axiom, path = rr.path, depth = rec_depth(c, rr);
     float sum = 0.0f;
     if (!is_static) {
+#pragma unroll kEntryUnroll<E>
         for (uint32_t i = 1; i < n; ++i) sum += P(c, e, i, rr, axiom, path, depth);
     } else {
         for (uint32_t i = n - 1; i >= 1; --i) {
@@ -165,6 +176,7 @@ __device__ __forceinline__ int32_t random_choice(const Ctx& c, const E& e, float
         }
     }
     float acc = 0.0f;
+#pragma unroll kEntryUnroll<E>
     for (uint32_t i = 1; i < n; ++i) {
         if (is_static && i == n - 1) return (int32_t)i - 1;
         float np = P(c, e, i, rr, axiom, path, depth) / sum;
@@ -408,6 +420,7 @@ struct Fan {
     float r2a;           // Subdivide: relative-to-absolute scale
     float off;           // running offset on the axis
     float e1, e2, e3;    // Repeat extents (start/mid/end)
+    float c1;            // Subdivide, constant entries: factor 0 as fan_init evaluated it (a draw is not cheap)
     float prev_ns;       // Subdivide: size and offset of the previous child
     float prev_o;
     uint32_t reps;       // Repeat repetitions
@@ -423,17 +436,18 @@ __device__ __forceinline__ void fan_init(const Ctx& c, const Rec& r, const E& e,
     f.r2a = 0.0f;
     f.off = 0.0f;
     f.e1 = f.e2 = f.e3 = 0.0f;
-    f.prev_ns = 0.0f; f.prev_o = 0.0f;
+    f.c1 = 0.0f; f.prev_ns = 0.0f; f.prev_o = 0.0f;
     if (kind == K_SUBDIV) {                    // Subdivide.cuh:142-153 / 181-216
         const uint32_t ax = r.axiom, pa = r.path, de = rec_depth(c, r);
         float abs_sum = 0.0f, rel_sum = 0.0f;
         uint32_t axis = 0;
-#pragma unroll 1
+#pragma unroll kEntryUnroll<E>
         for (uint32_t i = 0; i < e.nparams(); ++i) {
             float fac = P(c, e, i, r, ax, pa, de);
             if (i == 0) {
                 axis = f2u_rd(fac);
             } else {
+                if (E::kConst && i == 1) f.c1 = fac;
                 abs_sum += (float)(fac > 0.0f) * fac;
                 rel_sum += (float)(fac < 0.0f) * (fac * -1.0f);
             }
@@ -533,6 +547,8 @@ __device__ __forceinline__ bool fan_geom(const Ctx& c, const Rec& r, const E& e,
         float fac;
         if (p.type == PGA_PT_SCALAR) {
             fac = p.a;
+        } else if (E::kConst && j == 0u) {
+            fac = f.c1;                        // the same parameter of the same shape
         } else if (!is_static && j > 0 && shape_dependent(p.type)) {
             // the DynParams form evaluates factor j on the symbol that child
             // j-1 left behind (size, model and seed overwritten in place)
@@ -579,6 +595,7 @@ template <class E>
 __device__ __forceinline__ bool build_child(const Ctx& c, const Rec& r, const E& e, uint32_t j,
                                             uint32_t axis, float o, float ns, Rec& ch) {
     const uint32_t kind = e.kind();
+    axis = e.axis(axis);
     ch = r;
     if (kind == K_SUBDIV || kind == K_REPEAT) {
         if (c.geom) {

@@ -12,6 +12,7 @@
 // the specialised kernel computes the interpreter's instance records bit for
 // bit. Code objects are kept per process by a hash of their source, so
 // contexts that load the same program compile it once.
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
@@ -63,7 +64,8 @@ std::string fbits(float f) {
 
 }  // namespace
 
-std::string pga_spec_source(const std::vector<pga::DevEntry>& entries, uint32_t count_geom, uint32_t use_seed,
+std::string pga_spec_source(const std::vector<pga::DevEntry>& entries, const std::vector<pga::DevParam>& params,
+                            const std::vector<int32_t>& succ, uint32_t count_geom, uint32_t use_seed,
                             uint32_t block_size) {
     const size_t n = entries.size();
     std::vector<uint64_t> key(n);
@@ -106,7 +108,22 @@ std::string pga_spec_source(const std::vector<pga::DevEntry>& entries, uint32_t 
         s += "  static constexpr float pv0 = " + fbits(d.pv[0]) + ", pv1 = " + fbits(d.pv[1]) +
              ", pv2 = " + fbits(d.pv[2]) + ";\n";
         s += "  static constexpr int32_t sv0 = " + std::to_string(d.sv[0]) + ", sv1 = " + std::to_string(d.sv[1]) +
-             ", sv2 = " + std::to_string(d.sv[2]) + ";\n};\n";
+             ", sv2 = " + std::to_string(d.sv[2]) + ";\n";
+        // every parameter and successor (at least one, for the array's sake)
+        std::string pt, pa, pb, pc, sv;
+        for (uint32_t k = 0; k < std::max<uint32_t>(d.nparams, 1u); ++k) {
+            const pga::DevParam p = k < d.nparams && d.pbase + k < params.size() ? params[d.pbase + k] : pga::DevParam{};
+            const char* sep = k ? ", " : "";
+            pt += sep + std::to_string(p.type) + "u";
+            pa += sep + fbits(p.a);
+            pb += sep + fbits(p.b);
+            pc += sep + fbits(p.c);
+        }
+        for (uint32_t k = 0; k < std::max<uint32_t>(d.nsucc, 1u); ++k)
+            sv += (k ? ", " : "") + std::to_string(k < d.nsucc && d.sbase + k < succ.size() ? succ[d.sbase + k] : -1);
+        s += "  static constexpr uint32_t pt[] = {" + pt + "};\n";
+        s += "  static constexpr float pa[] = {" + pa + "}, pb[] = {" + pb + "}, pc[] = {" + pc + "};\n";
+        s += "  static constexpr int32_t sv[] = {" + sv + "};\n};\n";
     }
     s += "struct Prog {\n";
     bool polygons = false;   // a dynamic polygon or prism procedure: 6, 7, 14, 15

@@ -31,9 +31,11 @@
 namespace pga {
 
 // Fields every constant entry type shares, from D's constants idx, w0, w1,
-// pbase, sbase, pv0..pv2, sv0..sv2, aux0, aux1.
+// pbase, sbase, pv0..pv2, sv0..sv2, aux0, aux1 and the arrays of all its
+// parameters (pt, pa, pb, pc) and successors (sv).
 template <class D>
 struct SpecEntry {
+    static constexpr bool kConst = true;
     __device__ __forceinline__ static constexpr uint32_t kind() { return D::w0 & 0xFFu; }
     __device__ __forceinline__ static constexpr uint32_t shape() { return (D::w0 >> 8) & 0xFFu; }
     __device__ __forceinline__ static constexpr uint32_t flags() { return (D::w0 >> 16) & 0xFFu; }
@@ -49,7 +51,18 @@ struct SpecEntry {
         return k == 0u ? D::sv0 : (k == 1u ? D::sv1 : D::sv2);
     }
     __device__ __forceinline__ static uint32_t auxk(const Ctx&, uint32_t k) { return k == 0u ? D::aux0 : D::aux1; }
-    __device__ __forceinline__ static DevParam param(const Ctx& c, uint32_t k) { return c.prog.params[D::pbase + k]; }
+    // the loops over parameters and children are unrolled: k is a constant
+    __device__ __forceinline__ static DevParam param(const Ctx&, uint32_t k) {
+        return DevParam{D::pt[k], D::pa[k], D::pb[k], D::pc[k]};
+    }
+    __device__ __forceinline__ static int32_t svx(const Ctx&, uint32_t k) { return D::sv[k]; }
+    __device__ __forceinline__ static uint32_t axis(uint32_t a) {
+        if ((kind() == K_SUBDIV || kind() == K_REPEAT) && (inl() & 1u)) {
+            const uint32_t x = f2u_rd(D::pv0);
+            return x > 2u ? 0u : x;       // out of range: no children (Subdivide), axis 0 (Repeat)
+        }
+        return a;
+    }
 };
 
 // The entry type for an index outside the program (a dispatcher's default):
@@ -59,6 +72,9 @@ struct SpecNoEntry : SpecEntry<SpecNoEntry> {
     static constexpr uint32_t idx = 0u, w0 = K_NONE, w1 = 0u, pbase = 0u, sbase = 0u, aux0 = 0u, aux1 = 0u;
     static constexpr float pv0 = 0.0f, pv1 = 0.0f, pv2 = 0.0f;
     static constexpr int32_t sv0 = -1, sv1 = -1, sv2 = -1;
+    static constexpr uint32_t pt[1] = {0u};
+    static constexpr float pa[1] = {0.0f}, pb[1] = {0.0f}, pc[1] = {0.0f};
+    static constexpr int32_t sv[1] = {-1};
 };
 
 // An entry of a group: the entries of a program that share both header words
@@ -70,6 +86,7 @@ struct SpecNoEntry : SpecEntry<SpecNoEntry> {
 // operator forms rather than with the number of entries.
 template <uint32_t W0, uint32_t W1>
 struct SpecGroupEntry {
+    static constexpr bool kConst = false;
     static constexpr uint32_t w0 = W0, w1 = W1;
     uint32_t idx, pbase, sbase;
     float pv0, pv1, pv2;
@@ -88,6 +105,8 @@ struct SpecGroupEntry {
     }
     __device__ __forceinline__ uint32_t auxk(const Ctx& c, uint32_t k) const { return c.prog.entries[idx].aux[k]; }
     __device__ __forceinline__ DevParam param(const Ctx& c, uint32_t k) const { return c.prog.params[pbase + k]; }
+    __device__ __forceinline__ int32_t svx(const Ctx& c, uint32_t k) const { return c.prog.succ[sbase + k]; }
+    __device__ __forceinline__ uint32_t axis(uint32_t a) const { return a; }
     __device__ __forceinline__ static SpecGroupEntry at(const Ctx& c, uint32_t i) {
         const uint4* q = reinterpret_cast<const uint4*>(c.prog.entries) + i * 3u;
         const uint4 a = q[0], b = q[1];
@@ -112,6 +131,12 @@ __device__ __forceinline__ uint64_t spec_key(const Ctx& c, uint32_t i) {
     if (i >= S::kEntries) return K_NONE;
     const uint2 w = *reinterpret_cast<const uint2*>(c.prog.entries + i);
     return ((uint64_t)w.y << 32) | w.x;
+}
+
+// A 64-bit value that every lane holds, in scalar registers.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
+           __builtin_amdgcn_readfirstlane((uint32_t)v);
 }
 
 // Calls f(entry) for each lane with the entry of index `i` as its type: one
@@ -189,7 +214,7 @@ __device__ __forceinline__ void spec_pass(const KArgs& a, LevelLDS& L, float4* P
         uint32_t steps = 0, j = 0, dslot = 0, pidx = ~0u, fe = 0;
         uint32_t skipm = 0, nd = 0;
         Fan f;
-        f.n = 0; f.axis = 0; f.total = 0.0f; f.r2a = 0.0f; f.off = 0.0f;
+        f.n = 0; f.axis = 0; f.total = 0.0f; f.r2a = 0.0f; f.off = 0.0f; f.c1 = 0.0f;
         f.e1 = f.e2 = f.e3 = 0.0f; f.prev_ns = 0.0f; f.prev_o = 0.0f; f.reps = 0;
 #pragma unroll 1
         while (__ballot(mode != M_DONE) != 0ull) {
@@ -331,23 +356,17 @@ __device__ __forceinline__ void spec_pass(const KArgs& a, LevelLDS& L, float4* P
                     });
                 }
             }
-            if (__ballot(direct) != 0ull) {
-                // a direct lane is done with its own record (the parent is in
-                // PW): its children are built into `cur`
-#pragma unroll 1
-                for (uint32_t jj = 0; __ballot(direct && jj < f.n) != 0ull; ++jj) {
-                    uint32_t sl = 0;
-                    bool has = false;
-                    if (direct && jj < f.n)
-                        visit(c, fe, [&](const auto& e) {
-                            if (is_fanout(e.kind())) {
-                                const Rec par = par_load(PW);
-                                has = direct_child(c, par, e, f, skipm, jj, cur, sl);
-                            }
-                        });
-                    unsigned long long idx;
-                    emit_terminal(c, L, ST, true, has, sl, cur, idx);
-                }
+            // one entry of the wave's direct fan-outs after the other, with the
+            // whole wave (the entries of a group differ in their terminals)
+            unsigned long long pending = WR ? __ballot(direct) : 0ull;
+            while (pending != 0ull) {
+                const uint32_t u = __builtin_amdgcn_readlane(fe, __ffsll((long long)pending) - 1);
+                const bool mine = direct && fe == u;
+                auto all = [&](const auto& e) {
+                    if (e.flags() & EF_DIRECT) emit_direct(c, L, ST, PW, e, mine, f, skipm);
+                };
+                S::dispatch(c, uniform64(spec_key<S>(c, u)), u, all);
+                pending &= ~__ballot(mine);
             }
         }
     }
