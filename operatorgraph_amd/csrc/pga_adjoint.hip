@@ -58,7 +58,7 @@ __device__ __forceinline__ void grad_param(const Ctx& c, const AdjArgs& g, GradA
                                            uint32_t axiom, float v) {
     if (v == 0.0f || k >= e.nparams()) return;
     if (k < 3u && ((e.inl() >> k) & 1u)) return;
-    const DevParam p = c.prog.params[e.pbase + k];
+    const DevParam p = e.param(c, k);
     if (p.type != PGA_PT_AXIOM_PARAM || c.aparams_per == 0u) return;
     const uint32_t slot = (uint32_t)p.a;
     if (c.aparams_per <= kGradSlots && slot < kGradSlots && (ga.axiom == ~0u || ga.axiom == axiom)) {
@@ -298,43 +298,52 @@ __device__ __forceinline__ void build_adj(const Rec& p, const EntryV& pe, uint32
         float dt[3];
         translate_adj(p.m, t, dtmp, dp.m, dt);
         const float sgn = (j == 0 || j == 2 || j == 4) ? -0.5f : 0.5f;
-        const uint32_t ta = j < 2 ? 2u : (j < 4 ? 0u : 1u);
-        dp.s[ta] += sgn * dt[ta];
+        // (selects: an array indexed at run time lives in scratch)
+        const float dta = sgn * (j < 2 ? dt[2] : (j < 4 ? dt[0] : dt[1]));
+        dp.s[0] += j >= 2 && j < 4 ? dta : 0.0f;
+        dp.s[1] += j >= 4 ? dta : 0.0f;
+        dp.s[2] += j < 2 ? dta : 0.0f;
         // sizes: s_c = ((j == 2 || j == 3) ? sz : sx, j < 4 ? sy : sz, 1)
-        if (j == 2 || j == 3) dp.s[2] += dc.s[0]; else dp.s[0] += dc.s[0];
-        if (j < 4) dp.s[1] += dc.s[1]; else dp.s[2] += dc.s[1];
+        dp.s[2] += j == 2 || j == 3 ? dc.s[0] : 0.0f;
+        dp.s[0] += j == 2 || j == 3 ? 0.0f : dc.s[0];
+        dp.s[1] += j < 4 ? dc.s[1] : 0.0f;
+        dp.s[2] += j < 4 ? 0.0f : dc.s[1];
         return;
     }
     // K_REPLICATE: a copy
     dp = dc;
 }
 
-__device__ __forceinline__ const float* slot_at(const AdjArgs& g, uint32_t child) {
-    return g.slots + (size_t)child * kSlotFloats;
+__device__ __forceinline__ const float4* slot_at(const AdjArgs& g, uint32_t child) {
+    return g.slots + (size_t)child * (kSlotFloats / 4u);
 }
 
 // Reverse of a fan-out at state `r` (entry e), whose children's slots start
 // at child index `first` of the next level.
 __device__ __forceinline__ void fan_adj(const Ctx& c, const AdjArgs& g, GradAcc& ga, const EntryV& e, const Rec& r, uint32_t first,
                                         uint32_t nd, bool self, Adj& d) {
+    const uint32_t kind = e.kind();
+    const bool split = !self && (kind == K_SUBDIV || kind == K_REPEAT);
+    Fan f;
+    f.n = 0;
+    f.axis = 3u;
+    if (split) fan_init(c, r, e, f);
     // parent-state adjoints the children left (four 16-byte loads per slot),
     // and the sum of their offset adjoints in child order
     float total_o = 0.0f;
     for (uint32_t q = 0; q < nd; ++q) {
-        const float4* sl = reinterpret_cast<const float4*>(slot_at(g, first + q));
-        const float4 a = sl[0], b = sl[1], cc = sl[2], dd = sl[3];
+        const float4* sl = slot_at(g, first + q);
+        float4 a = sl[0], b = sl[1], cc = sl[2], dd = sl[3];
+        dd.x = f.axis == 0u ? 0.0f : dd.x;       // the child's size adjoint, below
+        dd.y = f.axis == 1u ? 0.0f : dd.y;
+        dd.z = f.axis == 2u ? 0.0f : dd.z;
         d.m[0] += a.x; d.m[1] += a.y; d.m[2] += a.z; d.m[3] += a.w;
         d.m[4] += b.x; d.m[5] += b.y; d.m[6] += b.z; d.m[7] += b.w;
         d.m[8] += cc.x; d.m[9] += cc.y; d.m[10] += cc.z; d.m[11] += cc.w;
         d.s[0] += dd.x; d.s[1] += dd.y; d.s[2] += dd.z;
         total_o += dd.w;
     }
-    if (self) return;
-    const uint32_t kind = e.kind();
-    if (kind != K_SUBDIV && kind != K_REPEAT) return;
-    Fan f;
-    fan_init(c, r, e, f);
-    if (f.n == 0u) return;
+    if (!split || f.n == 0u) return;
     uint32_t skipm = c.prog.entries[e.idx].aux[0];
     if (kind == K_REPEAT) skipm = (skipm & 1u) ? 0xFFFFFFFFu : 0u;
     // o_j = off_j + ns_j / 2, off_{j+1} = off_j + ns_j, off_0 = -total / 2:
@@ -348,7 +357,11 @@ __device__ __forceinline__ void fan_adj(const Ctx& c, const AdjArgs& g, GradAcc&
         const bool skip = j < 32u ? ((skipm >> j) & 1u) != 0u : skipm == 0xFFFFFFFFu;
         float d_oj = 0.0f, d_nsj = 0.0f;
         if (!skip) {
-            if (q < nd) { d_oj = slot_at(g, first + q)[15]; d_nsj = slot_at(g, first + q)[16]; }
+            if (q < nd) {
+                const float4 dd = slot_at(g, first + q)[3];
+                d_oj = dd.w;
+                d_nsj = f.axis == 0u ? dd.x : (f.axis == 1u ? dd.y : dd.z);
+            }
             ++q;
         }
         if (!keep) continue;
@@ -422,11 +435,36 @@ __device__ __forceinline__ void fan_adj(const Ctx& c, const AdjArgs& g, GradAcc&
     for (uint32_t q = 0; q < 3; ++q) d.s[q] = q == f.axis ? d.s[q] + d_total : d.s[q];
 }
 
-__device__ __forceinline__ Ctx adj_ctx(const KArgs& a) {
+// The program image and the tables a child looks up by terminal, in LDS: read
+// from global memory, every operator of every chain waited for its entry.
+struct AdjLDS {
+    unsigned long long cap[PGA_MAX_TERMINALS];
+    const float* dl[PGA_MAX_TERMINALS];
+};
+extern __shared__ __align__(16) unsigned char adj_smem[];
+
+__device__ __forceinline__ void adj_stage(const KArgs& a, const AdjArgs& g, AdjLDS& T) {
+    uint4* dst = reinterpret_cast<uint4*>(adj_smem);
+    for (uint32_t i = threadIdx.x; i < a.image_bytes / 16u; i += blockDim.x) dst[i] = a.image[i];
+    for (uint32_t i = threadIdx.x; i < PGA_MAX_TERMINALS; i += blockDim.x) {
+        T.cap[i] = a.inst_cap[i];
+        T.dl[i] = g.dl[i];
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ Ctx adj_ctx(const KArgs& a, const AdjLDS& T) {
     Ctx c;
-    c.prog = a.prog;
-    c.inst = a.inst;
-    c.inst_cap = a.inst_cap;
+    c.prog.entries = reinterpret_cast<const DevEntry*>(adj_smem);
+    c.prog.params = reinterpret_cast<const DevParam*>(adj_smem + a.off_params);
+    c.prog.succ = reinterpret_cast<const int32_t*>(adj_smem + a.off_succ);
+    c.prog.exp = reinterpret_cast<const uint32_t*>(adj_smem + a.off_exp);
+    c.prog.term_slot = adj_smem + a.off_slots;
+    c.prog.slot_term = adj_smem + a.off_slots + PGA_MAX_TERMINALS;
+    c.prog.nentries = a.prog.nentries;
+    c.prog.nslots = a.prog.nslots;
+    c.inst = nullptr;
+    c.inst_cap = T.cap;
     c.aparams = a.aparams;
     c.aparams_per = a.aparams_per;
     c.naxioms_total = a.naxioms_total;
@@ -445,7 +483,7 @@ __device__ __forceinline__ Ctx adj_ctx(const KArgs& a) {
     c.seed = a.use_seed;
     c.poly = 0u;             // the tape refuses dynamic polygons
     c.tape = 1u;
-    c.prog_lds = 0u;
+    c.prog_lds = 1u;
     c.ctxs = 0u;             // one-phase programs without Collider / IfCollides only
     c.dmask = 0xFFFFu;
     c.phase = 0u;
@@ -460,80 +498,109 @@ __device__ __forceinline__ Ctx adj_ctx(const KArgs& a) {
     return c;
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_adjoint(KArgs a, AdjArgs g) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.n_children) return;
-    const Ctx c = adj_ctx(a);
-    const uint32_t gi = g.child_base + i;
-    if (gi >= a.tape_out_cap || gi >= g.slots_cap) return;
-    float* my = g.slots + (size_t)gi * kSlotFloats;
-    const uint4 out = a.tape_out[gi];
-    const uint32_t kind = out.x & 0xFFu;
-    // the child's starting state
-    Rec s0, par;
-    uint32_t j = 0, axis = 0;
-    float o = 0.0f;
-    bool from_desc = false, self_copy = false;
+__device__ __forceinline__ void load_rec(const Rec* src, Rec& r) {
+    const float4* s = reinterpret_cast<const float4*>(src);
+    const float4 a = s[0], b = s[1], c = s[2], d = s[3], e = s[4];
+    r.m[0] = a.x; r.m[1] = a.y; r.m[2] = a.z; r.m[3] = a.w;
+    r.m[4] = b.x; r.m[5] = b.y; r.m[6] = b.z; r.m[7] = b.w;
+    r.m[8] = c.x; r.m[9] = c.y; r.m[10] = c.z; r.m[11] = c.w;
+    r.s[0] = d.x; r.s[1] = d.y; r.s[2] = d.z; r.seed = d.w;
+    r.custom = e.x; r.ed = __float_as_uint(e.y); r.axiom = __float_as_uint(e.z); r.path = __float_as_uint(e.w);
+}
+
+// A child's starting state: the axiom's record, or what its descriptor names.
+struct ChildRef {
+    uint4 dv;                           // descriptor (levels > 0)
+    uint32_t i;                         // child of the level
+};
+__device__ __forceinline__ void child_parent(const KArgs& a, const AdjArgs& g, const ChildRef& ch, Rec& par) {
+    load_rec(a.tape_par + g.par_in_base + ch.dv.x, par);
+}
+__device__ __forceinline__ void child_start(const KArgs& a, const AdjArgs& g, const Ctx& c, const ChildRef& ch,
+                                            Rec& r) {
     if (g.level == 0u) {
-        const pga_axiom& ax = a.axioms[a.first_axiom + i];
+        const pga_axiom& ax = a.axioms[a.first_axiom + ch.i];
 #pragma unroll
-        for (int k = 0; k < 12; ++k) s0.m[k] = ax.model[k];
-        s0.s[0] = ax.size[0]; s0.s[1] = ax.size[1]; s0.s[2] = ax.size[2];
-        s0.seed = ax.seed;
-        s0.custom = ax.custom;
-        s0.axiom = a.first_axiom + i;
-        s0.path = 0u;
-        s0.ed = (uint32_t)max(ax.entry_index, 0);
-    } else {
-        const uint4 dv = *reinterpret_cast<const uint4*>(a.tape_desc + g.desc_in_base + i);
-        const uint32_t jj = dv.y & 0x3FFFFFFFu;
-        if (kind == T_DROP || dv.x >= a.cap_par || jj == kDescNone) {
-#pragma unroll
-            for (uint32_t q = 0; q < kSlotFloats; ++q) my[q] = 0.0f;
-            return;
-        }
-        const Rec* pp = a.tape_par + g.par_in_base + dv.x;
-        par = *pp;
-        if (jj == kDescSelf) {
-            s0 = par;
-            self_copy = true;
-        } else {
-            j = jj;
-            axis = dv.y >> 30;
-            o = __uint_as_float(dv.z);
-            from_desc = true;
-            build_child(c, par, load_entry(c, rec_entry(par)), j, axis, o, __uint_as_float(dv.w), s0);
-        }
+        for (int k = 0; k < 12; ++k) r.m[k] = ax.model[k];
+        r.s[0] = ax.size[0]; r.s[1] = ax.size[1]; r.s[2] = ax.size[2];
+        r.seed = ax.seed;
+        r.custom = ax.custom;
+        r.axiom = a.first_axiom + ch.i;
+        r.path = 0u;
+        r.ed = (uint32_t)max(ax.entry_index, 0);
+        return;
     }
+    Rec par;
+    child_parent(a, g, ch, par);
+    const uint32_t j = ch.dv.y & 0x3FFFFFFFu;
+    if (j == kDescSelf) { r = par; return; }
+    build_child(c, par, load_entry(c, rec_entry(par)), j, ch.dv.y >> 30, __uint_as_float(ch.dv.z),
+                __uint_as_float(ch.dv.w), r);
+}
+
+// One thread per child of the level. What bounds it is the latency of a chain
+// of loads (outcome and descriptor, parent, its children's slots or its
+// instance's gradient) at few waves per SIMD, so registers: a thread holds
+// one record at a time and derives it again from the tape where it needs it
+// later (the parent is in L2), instead of the parent, the starting state and
+// the end of the chain side by side. Slots are 64 bytes and leave through LDS:
+// stored lane by lane, 312 MB of them became 716 MB of writes. The levels of
+// 4,096 parameterised lots, last first: 372 / 661 / 295 / 67 us with 80-byte
+// slots, the program read from memory and 48 bytes of scratch a lane; 299 /
+// 559 / 227 / 52 like this.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_adjoint(KArgs a, AdjArgs g) {
+    __shared__ AdjLDS T;
+    __shared__ float4 stage[4][256];     // per wave: 64 slots on their way out
+    adj_stage(a, g, T);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const Ctx c = adj_ctx(a, T);
+    const uint32_t gi = g.child_base + i;
+    const bool here = i < g.n_children && gi < a.tape_out_cap && gi < g.slots_cap;
+    uint4 out = make_uint4(T_DROP, 0u, 0u, 0u);
+    ChildRef ch;
+    ch.i = i;
+    ch.dv = make_uint4(0u, kDescNone, 0u, 0u);
+    if (here) {
+        out = a.tape_out[gi];
+        if (g.level != 0u) ch.dv = *reinterpret_cast<const uint4*>(a.tape_desc + g.desc_in_base + i);
+    }
+    const uint32_t jj = ch.dv.y & 0x3FFFFFFFu;
+    const bool none = g.level != 0u && (out.x == T_DROP || ch.dv.x >= a.cap_par || jj == kDescNone);
+    const uint32_t kind = none || !here ? (uint32_t)T_DROP : out.x & 0xFFu;
+    const bool self_copy = g.level != 0u && jj == kDescSelf;
     Adj d;
     adj_zero(d);
     GradAcc ga;
     grad_zero(ga);
     if (kind != T_DROP) {
         // replay the chain of single-child operators to its end
-        Rec r = s0;
         uint32_t steps = 0;
-        for (; steps < c.max_chain; ++steps) {
-            const EntryV e = load_entry(c, rec_entry(r));
-            if (!(e.kind() != K_GENERATE && e.kind() != K_DISCARD && !is_fanout(e.kind()))) break;
-            uint32_t ord;
-            const int32_t next = apply_single(c, e, r, &ord);
-            if (!advance(c, r, next, ord)) break;
-        }
-        // the adjoint of the chain's end
-        if (kind == T_TERM) {
-            const uint32_t slot = (out.x >> 8) & 0xFFu;
-            const uint32_t t = slot < c.prog.nslots ? c.prog.slot_term[slot] : PGA_MAX_TERMINALS;
-            if (t < PGA_MAX_TERMINALS && g.dl[t] != nullptr && (unsigned long long)out.y < a.inst_cap[t])
-                emit_adj(r, g.dl[t] + (size_t)out.y * 16u, d);
-        } else {   // T_FAN / T_SELF: the children of the fan-out are in the next level
-            const uint32_t first = g.next_child_base + out.z;
-            const uint32_t nd = first <= g.slots_cap && out.w <= g.slots_cap - first ? out.w : 0u;
-            fan_adj(c, g, ga, load_entry(c, rec_entry(r)), r, first, nd, kind == T_SELF, d);
+        {
+            Rec r;
+            child_start(a, g, c, ch, r);
+            for (; steps < c.max_chain; ++steps) {
+                const EntryV e = load_entry(c, rec_entry(r));
+                if (!(e.kind() != K_GENERATE && e.kind() != K_DISCARD && !is_fanout(e.kind()))) break;
+                uint32_t ord;
+                const int32_t next = apply_single(c, e, r, &ord);
+                if (!advance(c, r, next, ord)) break;
+            }
+            // the adjoint of the chain's end
+            if (kind == T_TERM) {
+                const uint32_t slot = (out.x >> 8) & 0xFFu;
+                const uint32_t t = slot < c.prog.nslots ? c.prog.slot_term[slot] : PGA_MAX_TERMINALS;
+                if (t < PGA_MAX_TERMINALS && T.dl[t] != nullptr && (unsigned long long)out.y < T.cap[t])
+                    emit_adj(r, T.dl[t] + (size_t)out.y * 16u, d);
+            } else {   // T_FAN / T_SELF: the children of the fan-out are in the next level
+                const uint32_t first = g.next_child_base + out.z;
+                const uint32_t nd = first <= g.slots_cap && out.w <= g.slots_cap - first ? out.w : 0u;
+                fan_adj(c, g, ga, load_entry(c, rec_entry(r)), r, first, nd, kind == T_SELF, d);
+            }
         }
         // back through the chain, recomputing each operator's input state
         for (uint32_t t = steps; t-- > 0;) {
-            Rec q = s0;
+            Rec q;
+            child_start(a, g, c, ch, q);
             for (uint32_t u = 0; u < t; ++u) {
                 const EntryV e = load_entry(c, rec_entry(q));
                 uint32_t ord;
@@ -547,15 +614,43 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     if (g.level == 0u) return;
     Adj dp;
     float d_o = 0.0f, d_ns = 0.0f;
-    if (self_copy) dp = d;
-    else if (from_desc) build_adj(par, load_entry(c, rec_entry(par)), j, axis, o, d, dp, d_o, d_ns);
-    else adj_zero(dp);
+    const uint32_t axis = ch.dv.y >> 30;
+    uint32_t pk = 0xFFu;
+    if (kind == T_DROP) {
+        adj_zero(dp);
+    } else if (self_copy) {
+        dp = d;
+    } else {
+        Rec par;
+        child_parent(a, g, ch, par);
+        const EntryV pe = load_entry(c, rec_entry(par));
+        pk = pe.kind();
+        build_adj(par, pe, ch.dv.y & 0x3FFFFFFFu, axis, __uint_as_float(ch.dv.z), d, dp, d_o, d_ns);
+    }
+    if (pk == K_SUBDIV || pk == K_REPEAT) {       // build_adj left 0 there
+        dp.s[0] = axis == 0u ? d_ns : dp.s[0];
+        dp.s[1] = axis == 1u ? d_ns : dp.s[1];
+        dp.s[2] = axis == 2u ? d_ns : dp.s[2];
+    }
+    // the wave's slots are consecutive: through LDS (record r's words rotated
+    // by r / 4 against bank conflicts) into whole lines
+    float4* S = stage[threadIdx.x >> 6];
+    const uint32_t lane = threadIdx.x & 63u;
+    auto at = [](uint32_t r, uint32_t k) { return r * 4u + ((k + (r >> 2)) & 3u); };
+    S[at(lane, 0u)] = make_float4(dp.m[0], dp.m[1], dp.m[2], dp.m[3]);
+    S[at(lane, 1u)] = make_float4(dp.m[4], dp.m[5], dp.m[6], dp.m[7]);
+    S[at(lane, 2u)] = make_float4(dp.m[8], dp.m[9], dp.m[10], dp.m[11]);
+    S[at(lane, 3u)] = make_float4(dp.s[0], dp.s[1], dp.s[2], d_o);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t n = (uint32_t)__popcll(__ballot(here));    // the lanes of `here` come first
+    float4* dst = g.slots + (size_t)(gi - lane) * (kSlotFloats / 4u);
 #pragma unroll
-    for (int k = 0; k < 12; ++k) my[k] = dp.m[k];
-    my[12] = dp.s[0]; my[13] = dp.s[1]; my[14] = dp.s[2];
-    my[15] = d_o;
-    my[16] = d_ns;
-    my[17] = my[18] = my[19] = 0.0f;
+    for (uint32_t u = 0; u < 4u; ++u) {
+        const uint32_t q = lane + 64u * u;
+        if (q < n * 4u) dst[q] = S[at(q >> 2, q & 3u)];
+    }
 }
 
 } // namespace pga
@@ -575,6 +670,6 @@ hipError_t pga_launch_grad_out(const double* acc, float* out, uint32_t n, hipStr
 
 hipError_t pga_launch_adjoint(const pga::KArgs& a, const pga::AdjArgs& g, hipStream_t s) {
     if (g.n_children == 0u) return hipSuccess;
-    hipLaunchKernelGGL(pga::k_adjoint, dim3((g.n_children + 255u) / 256u), dim3(256), 0, s, a, g);
+    hipLaunchKernelGGL(pga::k_adjoint, dim3((g.n_children + 255u) / 256u), dim3(256), a.image_bytes, s, a, g);
     return hipGetLastError();
 }

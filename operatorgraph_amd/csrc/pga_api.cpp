@@ -122,7 +122,6 @@ struct pga_context {
     pga::Desc* d_tape_desc = nullptr;
     uint4* d_tape_out = nullptr;
     float* d_adj_slots = nullptr;     // per child: the adjoint it leaves for its parent
-    const float** d_dl = nullptr;     // [PGA_MAX_TERMINALS] device table of dL/dinstance buffers
     double* d_grad64 = nullptr;       // FP64 accumulators of dL/dparams
     size_t grad64_cap = 0;
     uint32_t tape_par_cap = 0, tape_child_cap = 0, tape_blocks = 0;
@@ -1057,7 +1056,7 @@ PGA_API void pga_destroy(pga_context* ctx) {
     for (pga_graph* g : ctx->graphs) g->ctx = nullptr;   // the graphs stay valid to destroy
     hfree(ctx->d_image);
     hfree(ctx->d_tape_par); hfree(ctx->d_tape_desc); hfree(ctx->d_tape_out); hfree(ctx->d_adj_slots);
-    hfree(ctx->d_dl); hfree(ctx->d_grad64);
+    hfree(ctx->d_grad64);
     hfree(ctx->d_axioms_owned); hfree(ctx->d_aparams);
     hfree(ctx->d_inst_ptr); hfree(ctx->d_inst_cap);
     for (int b = 0; b < 2; ++b) { hfree(ctx->d_par[b]); hfree(ctx->d_desc[b]); }
@@ -1645,7 +1644,6 @@ PGA_API pga_status pga_tape_reserve(pga_context* ctx, uint32_t max_records, uint
     HIP_TRY(ctx, hipMalloc((void**)&ctx->d_tape_desc, (size_t)max_children * sizeof(pga::Desc)));
     HIP_TRY(ctx, hipMalloc((void**)&ctx->d_tape_out, (size_t)max_children * sizeof(uint4)));
     HIP_TRY(ctx, hipMalloc((void**)&ctx->d_adj_slots, (size_t)max_children * pga::kSlotFloats * sizeof(float)));
-    if (!ctx->d_dl) HIP_TRY(ctx, hipMalloc((void**)&ctx->d_dl, PGA_MAX_TERMINALS * sizeof(float*)));
     ctx->tape_par_cap = max_records;
     ctx->tape_child_cap = max_children;
     return PGA_OK;
@@ -1739,8 +1737,6 @@ PGA_API pga_status pga_backward(pga_context* ctx, const float* const* dl_dinstan
     for (uint32_t t = 0; t < PGA_MAX_TERMINALS; ++t)   // read as 16-byte rows
         if (((uintptr_t)dl_dinstances[t] & 15u) != 0u)
             return fail(ctx, PGA_ERR_INVALID_ARG, "dL/dinstance buffers must be 16-byte aligned");
-    HIP_TRY(ctx, hipMemcpyAsync((void*)ctx->d_dl, (const void*)dl_dinstances, PGA_MAX_TERMINALS * sizeof(float*),
-                                hipMemcpyHostToDevice, ctx->stream));
     const uint32_t n = ctx->tape_axioms;
     pga::KArgs a = make_args(ctx, 0, n);
     a.tape = 1;
@@ -1767,8 +1763,8 @@ PGA_API pga_status pga_backward(pga_context* ctx, const float* const* dl_dinstan
     HIP_TRY(ctx, hipMemsetAsync(ctx->d_grad64, 0, ng * sizeof(double), ctx->stream));
     for (uint32_t L = levels; L-- > 0;) {
         pga::AdjArgs g{};
-        g.dl = ctx->d_dl;
-        g.slots = ctx->d_adj_slots;
+        std::memcpy(g.dl, dl_dinstances, sizeof(g.dl));
+        g.slots = reinterpret_cast<float4*>(ctx->d_adj_slots);
         g.grad = ctx->d_grad64;
         g.level = L;
         g.n_children = L == 0 ? n : ctx->tape_dc[L - 1];

@@ -90,8 +90,10 @@ enum TapeKind : uint32_t { T_DROP = 0, T_TERM = 1, T_FAN = 2, T_SELF = 3 };
 
 // One level of the reverse pass.
 struct AdjArgs {
-    const float* const* dl;       // [PGA_MAX_TERMINALS] dL/dinstance (16 floats per instance) or null
-    float* slots;                 // per child: {dparent.m[12], dparent.s[3], d offset, d size, 0, 0, 0}
+    const float* dl[PGA_MAX_TERMINALS];   // dL/dinstance (16 floats per instance) or null
+    float4* slots;                // per child: {dparent.m[12], dparent.s[3], d offset}; a Subdivide's or Repeat's
+                                  // child keeps the adjoint of its size in s[axis], which its parent's size
+                                  // does not reach
     double* grad;                 // [axioms][params per axiom], FP64 accumulators
     uint32_t level;
     uint32_t n_children;          // children of this level
@@ -103,7 +105,7 @@ struct AdjArgs {
 };
 
 constexpr uint32_t kTapeBlock = 768;    // workgroup size of the tape-recording build (768 threads: 4.5 ms against 5.2 ms at 256 for Menger-5 with 16,384 parameterised lots)
-constexpr uint32_t kSlotFloats = 20;    // adjoint slot of a child (80 bytes)
+constexpr uint32_t kSlotFloats = 16;    // adjoint slot of a child (64 bytes)
 
 } // namespace pga
 
