@@ -347,3 +347,60 @@ def test_backward_refuses_a_replaced_tape():
             eng.backward(dl)
         assert e.value.status == abi.ERR_NOT_INITIALIZED
     eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 21, 43, 64])
+def test_adjoint_wave_edges_vs_fp64(n):
+    """Levels whose children end inside a wave (3 children a box face, the
+    adjoint's slots leave 64 at a time), every operator."""
+    _note(f"adjoint at the edges of a wave n={n}")
+    ax, params = _diff_axioms(n, seed=100 + n)
+    grad, ref, _ = _adjoint_pair(_diff_grammar(), ax, params, 3)
+    _assert_close(grad, ref)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 513, 512 * 512 - 1, 512 * 512 + 65])
+def test_fused_loss_tile_edges(n):
+    """The fused loss at the edges of a wave's tile, a workgroup and the
+    whole grid (then a workgroup takes a second tile), against FP64 torch."""
+    import torch
+    from operatorgraph_amd.autograd import center_size_mse, centers_and_sizes
+    _note(f"fused loss tiles n={n}")
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    inst = torch.randn(n, 16, generator=gen, device="cuda").requires_grad_(True)
+    tc = torch.randn(n, 3, generator=gen, device="cuda")
+    ts = torch.rand(n, 3, generator=gen, device="cuda")
+    loss = center_size_mse(inst, tc, ts, mean=False)
+    (g,) = torch.autograd.grad(loss, inst)
+    ref = inst.detach().double().requires_grad_(True)
+    c, s = centers_and_sizes(ref)
+    rl = ((c - tc) ** 2).sum() + ((s - ts) ** 2).sum()
+    (rg,) = torch.autograd.grad(rl, ref)
+    # FP32 terms of order 1 a row, summed in FP64
+    assert abs(loss.item() - rl.item()) <= 1e-5 * rl.item()
+    assert float((g - rg).abs().max()) <= 1e-5 * float(rg.abs().max())
+
+
+def test_axiom_params_from_device_tensors():
+    """Device tensors (any layout, float64 too) bind the same values as a
+    numpy array, and are copied before the call returns."""
+    import torch
+    from operatorgraph_amd import engine
+    _note("axiom parameters from device tensors")
+    ax, params = axioms.param_lots(24, perturb=0.05)
+    ref = _gpu_run(grammars.facade_params(), ax, params, 2, tape=False)
+    want = [ref.instances(t) for t in range(2)]
+    ref.close()
+    dev = torch.from_numpy(params).cuda()
+    forms = [dev.clone(), dev.double(), dev.t().contiguous().t(), torch.cat([dev, dev], dim=1)[:, :8]]
+    eng = engine.Engine(queue_capacity=1 << 20)
+    eng.load(grammars.facade_params()).set_axioms(ax)
+    for t in range(2):
+        eng.bind(t, 1 << 18)
+    for p in forms:
+        eng.set_axiom_params(p)
+        p.zero_()
+        eng.execute()
+        for t in range(2):
+            assert_same_multiset(eng.instances(t), want[t], f"terminal {t}")
+    eng.close()
