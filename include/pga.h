@@ -265,7 +265,8 @@ PGA_API pga_status pga_set_axioms_device(pga_context* ctx, const pga_axiom* devi
  * (n % 33) seeds into a 32-slot table, as the reference does. */
 PGA_API pga_status pga_set_seeds(pga_context* ctx, const float* seeds, uint32_t num_seeds);
 PGA_API pga_status pga_get_seeds(const pga_context* ctx, float* seeds32);
-/* per-axiom continuous parameters for PGA_PT_AXIOM_PARAM (host memory) */
+/* per-axiom continuous parameters for PGA_PT_AXIOM_PARAM, copied (host
+ * memory, or memory of the context's device that no other stream is writing) */
 PGA_API pga_status pga_set_axiom_params(pga_context* ctx, const float* params,
                                         uint32_t num_axioms, uint32_t params_per_axiom);
 PGA_API pga_status pga_set_philox_key(pga_context* ctx, uint32_t key0, uint32_t key1);

@@ -86,10 +86,14 @@ struct pga_context {
     pga::Rec* d_par[2] = {nullptr, nullptr};
     pga::Desc* d_desc[2] = {nullptr, nullptr};
     uint32_t cap = 0;
+    // what a run leaves for the host, one block (counter_bytes), read back in
+    // one copy: terminal counts, error word, per-level descriptor and parent
+    // counts (views)
     unsigned long long* d_term_counts = nullptr;
     uint32_t* d_par_counts = nullptr;
     uint32_t* d_desc_counts = nullptr;
     uint32_t* d_err = nullptr;
+    unsigned long long* h_counters = nullptr;   // pinned: the block, then the collider count
     uint32_t* d_bar = nullptr;
     uint32_t* d_block_totals = nullptr;
     uint64_t* ticks = nullptr;      // caller-owned timestamp buffer
@@ -981,6 +985,11 @@ pga_status status_from_err(pga_context* ctx, uint32_t err) {
 
 extern "C" {
 
+// The counter block in 4-byte words: 64 terminal counts, the error word (on a
+// line of its own), the per-level counts of max_levels + 2 levels each.
+static const uint32_t kErrWord = 2u * PGA_MAX_TERMINALS, kLevelWord = kErrWord + 16u;
+static size_t counter_words(const pga_context* ctx) { return kLevelWord + 2u * ((size_t)ctx->cfg.max_levels + 2u); }
+
 PGA_API uint32_t pga_abi_version(void) { return 1u; }
 
 PGA_API const char* pga_status_string(pga_status s) {
@@ -1035,11 +1044,13 @@ PGA_API pga_status pga_create(const pga_config* config, pga_context** out) {
     HIP_TRY(ctx, hipEventCreate(&ctx->ev1));
     HIP_TRY(ctx, hipEventCreate(&ctx->evk0));
     HIP_TRY(ctx, hipEventCreate(&ctx->evk1));
-    HIP_TRY(ctx, hipMalloc((void**)&ctx->d_term_counts, PGA_MAX_TERMINALS * sizeof(unsigned long long)));
-    HIP_TRY(ctx, hipMemset(ctx->d_term_counts, 0, PGA_MAX_TERMINALS * sizeof(unsigned long long)));
-    HIP_TRY(ctx, hipMalloc((void**)&ctx->d_par_counts, (ctx->cfg.max_levels + 2) * sizeof(uint32_t)));
-    HIP_TRY(ctx, hipMalloc((void**)&ctx->d_desc_counts, (ctx->cfg.max_levels + 2) * sizeof(uint32_t)));
-    HIP_TRY(ctx, hipMalloc((void**)&ctx->d_err, sizeof(uint32_t)));
+    const size_t words = counter_words(ctx);
+    HIP_TRY(ctx, hipMalloc((void**)&ctx->d_term_counts, words * sizeof(uint32_t)));
+    HIP_TRY(ctx, hipMemset(ctx->d_term_counts, 0, words * sizeof(uint32_t)));
+    HIP_TRY(ctx, hipHostMalloc((void**)&ctx->h_counters, (words + 2u) * sizeof(uint32_t), hipHostMallocDefault));
+    ctx->d_err = reinterpret_cast<uint32_t*>(ctx->d_term_counts) + kErrWord;
+    ctx->d_desc_counts = reinterpret_cast<uint32_t*>(ctx->d_term_counts) + kLevelWord;
+    ctx->d_par_counts = ctx->d_desc_counts + ctx->cfg.max_levels + 2u;
     HIP_TRY(ctx, hipMalloc((void**)&ctx->d_bar, pga::kBarWords * sizeof(uint32_t)));
     HIP_TRY(ctx, hipMemset(ctx->d_bar, 0, pga::kBarWords * sizeof(uint32_t)));
     HIP_TRY(ctx, hipMalloc((void**)&ctx->d_inst_ptr, PGA_MAX_TERMINALS * sizeof(pga_instance*)));
@@ -1060,11 +1071,11 @@ PGA_API void pga_destroy(pga_context* ctx) {
     hfree(ctx->d_axioms_owned); hfree(ctx->d_aparams);
     hfree(ctx->d_inst_ptr); hfree(ctx->d_inst_cap);
     for (int b = 0; b < 2; ++b) { hfree(ctx->d_par[b]); hfree(ctx->d_desc[b]); }
-    hfree(ctx->d_term_counts); hfree(ctx->d_par_counts); hfree(ctx->d_desc_counts);
-    hfree(ctx->d_err); hfree(ctx->d_bar); hfree(ctx->d_block_totals); hfree(ctx->d_loc);
+    hfree(ctx->d_term_counts); hfree(ctx->d_bar); hfree(ctx->d_block_totals); hfree(ctx->d_loc);
     hfree(ctx->d_coll); hfree(ctx->d_coll_count); hfree(ctx->d_coll_bits);
     drop_collider_bvh(ctx);
     if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
+    if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->evk0) (void)hipEventDestroy(ctx->evk0);
@@ -1136,7 +1147,17 @@ PGA_API pga_status pga_set_axiom_params(pga_context* ctx, const float* params, u
         HIP_TRY(ctx, hipMalloc((void**)&ctx->d_aparams, bytes));
         ctx->aparams_cap = bytes;
     }
-    if (bytes) HIP_TRY(ctx, hipMemcpy(ctx->d_aparams, params, bytes, hipMemcpyHostToDevice));
+    // values on this device are copied there, after the work on the context's
+    // stream; either way the caller's array may change once this returns
+    hipPointerAttribute_t at{};
+    const bool known = bytes && hipPointerGetAttributes(&at, params) == hipSuccess;
+    if (bytes && !known) (void)hipGetLastError();
+    if (known && at.type == hipMemoryTypeDevice && at.device == ctx->device) {
+        HIP_TRY(ctx, hipMemcpyAsync(ctx->d_aparams, params, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    } else if (bytes) {
+        HIP_TRY(ctx, hipMemcpy(ctx->d_aparams, params, bytes, known ? hipMemcpyDefault : hipMemcpyHostToDevice));
+    }
     ctx->aparams_per = per_axiom;
     ctx->aparams_axioms = num_axioms;
     return PGA_OK;
@@ -1162,10 +1183,10 @@ PGA_API pga_status pga_bind_instances(pga_context* ctx, uint32_t terminal, pga_i
 PGA_API pga_status pga_get_counts(pga_context* ctx, uint64_t* counts, uint32_t n) {
     if (!ctx || !counts || n > PGA_MAX_TERMINALS) return fail(ctx, PGA_ERR_INVALID_ARG, "bad counts request");
     NO_CAPTURE(ctx, "pga_get_counts");
-    unsigned long long tmp[PGA_MAX_TERMINALS];
-    HIP_TRY(ctx, hipMemcpyAsync(tmp, ctx->d_term_counts, sizeof(tmp), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipMemcpyAsync(ctx->h_counters, ctx->d_term_counts, PGA_MAX_TERMINALS * sizeof(unsigned long long),
+                                hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    for (uint32_t i = 0; i < n; ++i) counts[i] = tmp[i];
+    for (uint32_t i = 0; i < n; ++i) counts[i] = ctx->h_counters[i];
     return PGA_OK;
 }
 
@@ -1185,22 +1206,29 @@ static pga_status check_launch(pga_context* ctx, uint32_t first, uint32_t count)
     return ensure_buffers(ctx);
 }
 
-// Reads the error word, level and terminal counters of the finished run.
+// Enqueues the copy of the counters to the host, in place of a blocking copy
+// of each one after the run (five of about 25 us).
+static pga_status fetch_counters(pga_context* ctx) {
+    const size_t words = counter_words(ctx);
+    HIP_TRY(ctx, hipMemcpyAsync(ctx->h_counters, ctx->d_term_counts, words * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                ctx->stream));
+    if (ctx->collision && ctx->d_coll_count)
+        HIP_TRY(ctx, hipMemcpyAsync(reinterpret_cast<uint32_t*>(ctx->h_counters) + words, ctx->d_coll_count,
+                                    sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    return PGA_OK;
+}
+
+// Stats and status of a finished run from the fetched counters.
 static pga_status finish(pga_context* ctx, uint32_t count, uint32_t host_levels) {
-    uint32_t err = 0;
-    HIP_TRY(ctx, hipMemcpy(&err, ctx->d_err, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    std::vector<uint32_t> lc(ctx->cfg.max_levels + 2), pc(ctx->cfg.max_levels + 2);
-    HIP_TRY(ctx, hipMemcpy(lc.data(), ctx->d_desc_counts, lc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(pc.data(), ctx->d_par_counts, pc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    unsigned long long tc[PGA_MAX_TERMINALS];
-    HIP_TRY(ctx, hipMemcpy(tc, ctx->d_term_counts, sizeof(tc), hipMemcpyDeviceToHost));
+    const uint32_t* hw = reinterpret_cast<const uint32_t*>(ctx->h_counters);
+    uint32_t err = hw[kErrWord];
+    const uint32_t* lc = hw + kLevelWord;
+    const uint32_t* pc = lc + ctx->cfg.max_levels + 2u;
+    const unsigned long long* tc = ctx->h_counters;
     uint32_t levels = host_levels;
     if (ctx->cfg.technique == PGA_TECHNIQUE_MEGAKERNEL && count > 0) levels = lc[ctx->cfg.max_levels + 1];
     ctx->colliders = 0;
-    if (ctx->collision && ctx->d_coll_count) {
-        HIP_TRY(ctx, hipMemcpy(&ctx->colliders, ctx->d_coll_count, sizeof(uint32_t), hipMemcpyDeviceToHost));
-        ctx->colliders = std::min(ctx->colliders, ctx->coll_cap);
-    }
+    if (ctx->collision && ctx->d_coll_count) ctx->colliders = std::min(hw[counter_words(ctx)], ctx->coll_cap);
     // the specialised kernel's workgroup-local levels: the deepest and the
     // parent records they wrote
     ctx->stats.levels = std::max(levels, pc[ctx->cfg.max_levels + 1]);
@@ -1302,6 +1330,7 @@ PGA_API pga_status pga_execute_async(pga_context* ctx, uint32_t first, uint32_t 
 PGA_API pga_status pga_synchronize(pga_context* ctx) {
     if (!ctx) return PGA_ERR_INVALID_ARG;
     NO_CAPTURE(ctx, "pga_synchronize");
+    if (pga_status st = fetch_counters(ctx)) return st;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     float ms = 0.0f;
     HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->evk0, ctx->evk1));
@@ -1352,6 +1381,7 @@ PGA_API pga_status pga_execute_range(pga_context* ctx, uint32_t first, uint32_t 
     }
     HIP_TRY(ctx, hipEventRecord(ctx->evk1, ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    if ((st = fetch_counters(ctx))) return st;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     float ms = 0.0f;
     HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -1678,6 +1708,7 @@ PGA_API pga_status pga_forward_tape(pga_context* ctx, uint32_t num_axioms, doubl
     if (num_axioms > 0) HIP_TRY(ctx, pga_launch_mega_tape(a, ctx->tape_blocks, ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->evk1, ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    if ((st = fetch_counters(ctx))) return st;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     float ms = 0.0f;
     HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -1685,20 +1716,18 @@ PGA_API pga_status pga_forward_tape(pga_context* ctx, uint32_t num_axioms, doubl
     if (seconds) *seconds = ms * 1e-3;
     // per-level counts of the tape (the stats' queue check uses the ping-pong
     // capacity, the tape its own)
-    uint32_t err = 0;
-    HIP_TRY(ctx, hipMemcpy(&err, ctx->d_err, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    std::vector<uint32_t> lc(ctx->cfg.max_levels + 2), pc(ctx->cfg.max_levels + 2);
-    HIP_TRY(ctx, hipMemcpy(lc.data(), ctx->d_desc_counts, lc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    HIP_TRY(ctx, hipMemcpy(pc.data(), ctx->d_par_counts, pc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    unsigned long long tc[PGA_MAX_TERMINALS];
-    HIP_TRY(ctx, hipMemcpy(tc, ctx->d_term_counts, sizeof(tc), hipMemcpyDeviceToHost));
+    const uint32_t* hw = reinterpret_cast<const uint32_t*>(ctx->h_counters);
+    uint32_t err = hw[kErrWord];
+    const uint32_t* lc = hw + kLevelWord;
+    const uint32_t* pc = lc + ctx->cfg.max_levels + 2u;
+    const unsigned long long* tc = ctx->h_counters;
     const uint32_t levels = num_axioms ? lc[ctx->cfg.max_levels + 1] : 0u;
     ctx->stats.levels = levels;
     ctx->stats.records = 0;
     ctx->stats.terminals = 0;
     for (int t = 0; t < PGA_MAX_TERMINALS; ++t) ctx->stats.terminals += tc[t];
-    ctx->tape_pc.assign(pc.begin(), pc.begin() + levels);
-    ctx->tape_dc.assign(lc.begin(), lc.begin() + levels);
+    ctx->tape_pc.assign(pc, pc + levels);
+    ctx->tape_dc.assign(lc, lc + levels);
     uint64_t sp = 0, sd = 0;
     for (uint32_t l = 0; l < levels; ++l) { sp += pc[l]; sd += lc[l]; }
     ctx->stats.records = sp;
@@ -1777,13 +1806,12 @@ PGA_API pga_status pga_backward(pga_context* ctx, const float* const* dl_dinstan
     }
     HIP_TRY(ctx, pga_launch_grad_out(ctx->d_grad64, dl_dparams, (uint32_t)ng, ctx->stream));
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
+    HIP_TRY(ctx, hipMemcpyAsync(ctx->h_pinned, ctx->d_err, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     float ms = 0.0f;
     HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     if (seconds) *seconds = ms * 1e-3;
-    uint32_t err = 0;
-    HIP_TRY(ctx, hipMemcpy(&err, ctx->d_err, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    return status_from_err(ctx, err);
+    return status_from_err(ctx, ctx->h_pinned[0]);
 }
 
 PGA_API pga_status pga_capture_begin(pga_context* ctx) {

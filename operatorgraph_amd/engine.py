@@ -124,6 +124,7 @@ class Engine:
         st = self.L.pga_create(C.byref(cfg), C.byref(h))
         self._h = h.value
         self._check(st)
+        self._device = torch.cuda.current_device()   # pga_create made `device` current
         self._keep = {}
         self._ext = None
         self._capturing = False
@@ -196,6 +197,17 @@ class Engine:
         return self
 
     def set_axiom_params(self, params):
+        """(axioms, params per axiom) values, copied before the call returns: a
+        numpy array or a torch tensor, which stays on the device if it is on
+        the engine's."""
+        torch = self.torch
+        if isinstance(params, torch.Tensor) and params.is_cuda and \
+                params.device.index == torch.cuda.current_device() == self._device:
+            p = params.detach().to(torch.float32).contiguous()
+            self._after_torch()
+            self._check(self.L.pga_set_axiom_params(self._h, C.c_void_p(p.data_ptr()), p.shape[0], p.shape[1]))
+            self.params_per_axiom = p.shape[1]
+            return self
         if hasattr(params, "detach"):
             params = params.detach().cpu().numpy()
         p = np.ascontiguousarray(params, dtype=np.float32)
