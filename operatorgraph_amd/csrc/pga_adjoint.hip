@@ -492,7 +492,8 @@ __device__ __forceinline__ Ctx adj_ctx(const KArgs& a, const AdjLDS& T) {
     c.coll_count = nullptr;
     c.coll_visible = nullptr;
     c.coll_cap = 0u;
-    c.bvh_flat = nullptr;
+    c.bvh_wide = nullptr;
+    c.bvh_keys = nullptr;
     c.coll_bits = nullptr;
     c.coll_bits_cap = 0u;
     return c;

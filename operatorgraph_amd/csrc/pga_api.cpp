@@ -117,7 +117,7 @@ struct pga_context {
     uint64_t* d_coll_keys = nullptr;
     int32_t* d_coll_tree = nullptr;   // left | right | parent | leaf parent, coll_bvh_cap each
     float* d_coll_nodes = nullptr;
-    float4* d_coll_flat = nullptr;    // the tree in depth-first order, 2 coll_bvh_cap - 1 nodes
+    float4* d_coll_wide = nullptr;    // the tree four-wide, coll_bvh_cap - 1 nodes of eight words
     uint32_t* d_coll_bits = nullptr;  // per child of a level: IfCollides outcomes of the count pass
     uint32_t coll_bits_n = 0;
 
@@ -794,7 +794,7 @@ void drop_collider_bvh(pga_context* ctx) {
     hfree(ctx->d_coll_keys);
     hfree(ctx->d_coll_tree);
     hfree(ctx->d_coll_nodes);
-    hfree(ctx->d_coll_flat);
+    hfree(ctx->d_coll_wide);
 }
 
 // The collider store of a program with Collider / IfCollides (coll_cap_req
@@ -836,7 +836,7 @@ pga_status ensure_colliders(pga_context* ctx) {
     if (e == hipSuccess) e = hipMalloc((void**)&ctx->d_coll_keys, (size_t)want * sizeof(uint64_t));
     if (e == hipSuccess) e = hipMalloc((void**)&ctx->d_coll_tree, (size_t)want * 4u * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc((void**)&ctx->d_coll_nodes, (size_t)want * 6u * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc((void**)&ctx->d_coll_flat, (size_t)want * 2u * 2u * sizeof(float4));
+    if (e == hipSuccess) e = hipMalloc((void**)&ctx->d_coll_wide, (size_t)want * 8u * sizeof(float4));
     ctx->coll_bvh = b;
     if (e != hipSuccess) {
         drop_collider_bvh(ctx);
@@ -1282,9 +1282,10 @@ static pga_status begin_phase(pga_context* ctx, pga::KArgs& a, uint32_t p) {
         const uint32_t c = ctx->coll_bvh_cap;
         int32_t* t = ctx->d_coll_tree;
         HIP_TRY(ctx, pga_lbvh_enqueue_counted(ctx->coll_bvh, ctx->d_coll_boxes, ctx->d_coll_count, ctx->d_coll_keys,
-                                              t, t + c, t + 2u * c, t + 3u * c, ctx->d_coll_nodes,
-                                              ctx->d_coll_flat));
-        a.bvh_flat = ctx->d_coll_flat;
+                                              t, t + c, t + 2u * c, t + 3u * c, ctx->d_coll_nodes, ctx->d_coll,
+                                              ctx->d_coll_wide));
+        a.bvh_wide = ctx->d_coll_wide;
+        a.bvh_keys = reinterpret_cast<const unsigned long long*>(ctx->d_coll_keys);
     }
     HIP_TRY(ctx, pga_launch_reset(a, 2, ctx->stream));
     return PGA_OK;

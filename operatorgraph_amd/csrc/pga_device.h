@@ -140,10 +140,11 @@ struct Ctx {
     uint32_t* coll_count;
     const uint32_t* coll_visible;
     uint32_t coll_cap;
-    // linear BVH over the visible colliders in depth-first order (NULL: none
-    // built): per node two 16-byte words, box min xyz, max x | max y, max z,
-    // the node after its subtree, the collider of a leaf (~0: internal)
-    const float4* bvh_flat;
+    // linear BVH over the visible colliders, four children a node (NULL: none
+    // built): eight 16-byte words per binary node, see kWideLeaf; and the
+    // sorted keys of its leaves (collider = low word)
+    const float4* bvh_wide;
+    const unsigned long long* bvh_keys;
     // per child of the level: the IfCollides outcomes of the count pass, bit
     // k for the child's k-th IfCollides (k < 32), replayed by the write pass
     uint32_t* coll_bits;
@@ -157,7 +158,21 @@ struct CollMemo {
     uint32_t bits;
     uint32_t n;        // IfCollides met so far
     uint32_t mode;     // 0: neither, 1: record, 2: replay
+    // the lane's stack for BVH walks: kWalkStack words in LDS, word k at
+    // stack[(k / 4) * stride + k % 4] (the place of its fan-out parent, which
+    // it has none of while it runs a chain with an IfCollides in it)
+    __attribute__((address_space(3))) uint32_t* stack;
+    uint32_t stride;
 };
+constexpr uint32_t kWalkStack = 20u;
+
+// Node i of the four-wide BVH: the children of its children (or its children,
+// where those are leaves), their boxes as min x, y, z, max x, y, z of all four,
+// then their references - a leaf's collider | kWideLeaf, a node's index,
+// kWideNone for an absent one - and the node's own sorted leaf range
+// [first, last + 1) with the low 16 bits of the four leaves' tags, so that a
+// leaf of another tag is passed by without a look at its collider.
+constexpr uint32_t kWideLeaf = 0x80000000u, kWideNone = 0xFFFFFFFFu;
 
 // Axis-aligned box around a Box or Quad shape (a Quad with its z extent,
 // which the collision test keeps on the Quad's own face axis) under its

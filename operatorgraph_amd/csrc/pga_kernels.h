@@ -64,7 +64,8 @@ struct KArgs {
     uint32_t* coll_count;
     const uint32_t* coll_visible;
     uint32_t coll_cap;
-    const float4* bvh_flat;             // BVH over the visible colliders, depth-first (NULL: none)
+    const float4* bvh_wide;             // BVH over the visible colliders, four-wide (NULL: none)
+    const unsigned long long* bvh_keys; // the sorted keys of its leaves
     uint32_t* coll_bits;                // per child of a level: IfCollides outcomes of the count pass
     uint32_t coll_bits_cap;
     // derivation tape (reverse mode): every level's parent records and
@@ -130,11 +131,11 @@ hipError_t pga_launch_mega_tape(const pga::KArgs& a, uint32_t blocks, hipStream_
 hipError_t pga_launch_collider_boxes(const float4* coll, uint32_t cap, const uint32_t* count, float* aabbs,
                                      hipStream_t s);
 // the LBVH build over a device count word: leaves min(*nd, capacity), scene
-// box from the device, then the tree in depth-first order with skip indices
-// (2 * capacity - 1 nodes of two float4 in `flat`; pga_lbvh.hip)
+// box from the device, then the tree four-wide over the colliders `coll`
+// (capacity - 1 nodes of eight float4 in `wide`; pga_lbvh.hip)
 hipError_t pga_lbvh_enqueue_counted(pga_lbvh* b, const float* aabbs, const uint32_t* nd, uint64_t* keys,
                                     int32_t* left, int32_t* right, int32_t* parent, int32_t* leaf_parent,
-                                    float* node_aabb, float4* flat);
+                                    float* node_aabb, const float4* coll, float4* wide);
 hipError_t pga_launch_adjoint(const pga::KArgs& a, const pga::AdjArgs& g, hipStream_t s);
 hipError_t pga_launch_grad_out(const double* acc, float* out, uint32_t n, hipStream_t s);
 #endif

@@ -60,6 +60,8 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
         CollMemo memo;                  // context-sensitive kernels: IfCollides outcomes, count -> write pass
         memo.bits = 0u;
         memo.n = 0u;
+        memo.stack = (__attribute__((address_space(3))) uint32_t*)(PW + threadIdx.x);
+        memo.stride = 4u * blockDim.x;
         memo.mode = (CS && valid && i < c.coll_bits_cap) ? (wr ? 2u : 1u) : 0u;
         if (CS && memo.mode == 2u) memo.bits = c.coll_bits[i];
         uint32_t out_kind = T_DROP, out_a = 0, out_b = 0, out_c = 0;   // tape outcome

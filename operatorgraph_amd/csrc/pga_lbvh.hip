@@ -769,53 +769,57 @@ __global__ void __launch_bounds__(kThreads) k_tree_roots(const u64* __restrict__
     leave_roots(T, &I, 0u, m, roots + (size_t)blockIdx.x * kMaxRoots, nroots + blockIdx.x);
 }
 
-// The tree in depth-first order with skip indices, for walks without a
-// stack: node k is two float4, box min xyz, max x | max y, max z, the index
-// after k's subtree, the box index of a leaf (0xFFFFFFFF: internal). The
-// node whose sorted leaf range starts at a sits at 2a + (the number of its
-// ancestors whose left subtree holds it): the subtrees to its left hold a
-// leaves and a - (ancestors it is the right child of) internal nodes, and
-// each ancestor comes before it. Its subtree spans 2 (leaves) - 1 nodes.
-// Thread t < n: leaf t; n <= t < 2n - 1: internal node t - n.
-__global__ void __launch_bounds__(256) k_flatten(const unsigned long long* __restrict__ keys, uint32_t n,
-                                                 const uint32_t* nd, const int32_t* __restrict__ left,
-                                                 const int32_t* __restrict__ parent,
-                                                 const int32_t* __restrict__ leaf_parent,
-                                                 const int32_t* __restrict__ other_end,
-                                                 const float* __restrict__ node_aabb,
-                                                 const float* __restrict__ aabbs, float4* __restrict__ flat) {
+// The tree with four children a node, for walks (collider_hit): binary node i
+// takes its children's children, or a child itself where it is a leaf. One
+// thread per binary node (a walk from the root meets those at even depths).
+__global__ void __launch_bounds__(256) k_wide(const u64* __restrict__ keys, uint32_t n, const uint32_t* nd,
+                                              const int32_t* __restrict__ left, const int32_t* __restrict__ right,
+                                              const int32_t* __restrict__ other_end,
+                                              const float* __restrict__ node_aabb, const float* __restrict__ aabbs,
+                                              const float4* __restrict__ coll, float4* __restrict__ wide) {
     const uint32_t nn = leaf_count(n, nd);
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (nn == 0u || t >= 2u * nn - 1u) return;
-    int32_t cur, par;
-    uint32_t first, len, item;
-    const float* box;
-    if (t < nn) {
-        cur = (int32_t)t;
-        par = nn > 1u ? leaf_parent[t] : -1;
-        first = t;
-        len = 1u;
-        item = (uint32_t)keys[t];
-        box = aabbs + (size_t)item * 6u;
-    } else {
-        const int32_t j = (int32_t)(t - nn);
-        const int32_t e = other_end[j];
-        cur = -j;
-        par = j == 0 ? -1 : parent[j];
-        first = (uint32_t)min(j, e);
-        len = 2u * ((uint32_t)max(j, e) - first + 1u) - 1u;
-        item = 0xFFFFFFFFu;
-        box = node_aabb + (size_t)j * 6u;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (nn < 2u || i >= nn - 1u) return;
+    float b[4][6];
+    uint32_t ref[4], tag[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int32_t c = h == 0 ? left[i] : right[i];
+        int32_t g[2] = {c, 0};           // the slots' subtrees
+        bool two = false;
+        if (c < 0) {
+            g[0] = left[-c];
+            g[1] = right[-c];
+            two = true;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int q = 2 * h + k;
+            const bool there = k == 0 || two;
+            const float* src = nullptr;
+            ref[q] = 0xFFFFFFFFu;        // kWideNone
+            tag[q] = 0u;
+            if (there && g[k] >= 0) {
+                const uint32_t item = (uint32_t)keys[g[k]];
+                ref[q] = item | 0x80000000u;        // kWideLeaf
+                tag[q] = __float_as_uint(coll[(size_t)item * 5u + 3u].w) & 0xFFFFu;
+                src = aabbs + (size_t)item * 6u;
+            } else if (there) {
+                ref[q] = (uint32_t)-g[k];
+                src = node_aabb + (size_t)(-g[k]) * 6u;
+            }
+#pragma unroll
+            for (int z = 0; z < 6; ++z) b[q][z] = there ? src[z] : (z < 3 ? INFINITY : -INFINITY);
+        }
     }
-    uint32_t lefts = 0;
-    while (par >= 0) {                     // at most the tree's depth
-        if (left[par] == cur) ++lefts;
-        cur = -par;
-        par = parent[par];
-    }
-    const uint32_t k = 2u * first + lefts;
-    flat[2u * k] = make_float4(box[0], box[1], box[2], box[3]);
-    flat[2u * k + 1u] = make_float4(box[4], box[5], __uint_as_float(k + len), __uint_as_float(item));
+    float4* o = wide + (size_t)i * 8u;
+#pragma unroll
+    for (int z = 0; z < 6; ++z) o[z] = make_float4(b[0][z], b[1][z], b[2][z], b[3][z]);
+    o[6] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
+                       __uint_as_float(ref[3]));
+    const uint32_t e = (uint32_t)other_end[i];
+    o[7] = make_float4(__uint_as_float(min(i, e)), __uint_as_float(max(i, e) + 1u),
+                       __uint_as_float(tag[0] | tag[1] << 16), __uint_as_float(tag[2] | tag[3] << 16));
 }
 
 } // namespace bvhk
@@ -1117,7 +1121,7 @@ PGA_API pga_status pga_lbvh_build_device(pga_lbvh* b, const float* aabbs, const 
 // min(*nd, capacity) leaves, the scene box from the device.
 hipError_t pga_lbvh_enqueue_counted(pga_lbvh* b, const float* aabbs, const uint32_t* nd, uint64_t* keys,
                                     int32_t* left, int32_t* right, int32_t* parent, int32_t* leaf_parent,
-                                    float* node_aabb, float4* flat) {
+                                    float* node_aabb, const float4* coll, float4* wide) {
     const uint32_t n = b->capacity;
     const uint32_t blocks = std::min<uint32_t>(1024u, (n + 255u) / 256u);
     hipLaunchKernelGGL(k_bounds, dim3(blocks), dim3(256), 0, b->stream, aabbs, n, nd, b->bounds);
@@ -1126,9 +1130,8 @@ hipError_t pga_lbvh_enqueue_counted(pga_lbvh* b, const float* aabbs, const uint3
     const hipError_t e = enqueue_build(b->scratch, b->stream, aabbs, n, nd, zero, one, b->bounds, keys, left, right,
                                        parent, leaf_parent, node_aabb, b->other_end);
     if (e != hipSuccess) return e;
-    const uint32_t g = (uint32_t)(((uint64_t)2u * n + 255u) / 256u);
-    hipLaunchKernelGGL(k_flatten, dim3(g), dim3(256), 0, b->stream, reinterpret_cast<const unsigned long long*>(keys),
-                       n, nd, left, parent, leaf_parent, b->other_end, node_aabb, aabbs, flat);
+    hipLaunchKernelGGL(k_wide, dim3(ceil_div(n, 256u)), dim3(256), 0, b->stream, reinterpret_cast<const u64*>(keys), n,
+                       nd, left, right, b->other_end, node_aabb, aabbs, coll, wide);
     return hipGetLastError();
 }
 

@@ -397,7 +397,8 @@ __device__ __forceinline__ Ctx make_ctx(const KArgs& a, const LevelLDS& L, uint3
     c.coll_count = CS ? a.coll_count : nullptr;
     c.coll_visible = CS ? a.coll_visible : nullptr;
     c.coll_cap = CS ? a.coll_cap : 0u;
-    c.bvh_flat = CS ? a.bvh_flat : nullptr;
+    c.bvh_wide = CS ? a.bvh_wide : nullptr;
+    c.bvh_keys = CS ? a.bvh_keys : nullptr;
     c.coll_bits = CS ? a.coll_bits : nullptr;
     c.coll_bits_cap = CS ? a.coll_bits_cap : 0u;
     return c;

@@ -237,8 +237,23 @@ __device__ __forceinline__ bool shapes_overlap(const float am[12], const float a
     const float bh[3] = {bs[0] * 0.5f, bs[1] * 0.5f, bs[2] * 0.5f};
     const float aq[3] = {ah[0], ah[1], 0.0f}, bq[3] = {bh[0], bh[1], 0.0f};
     const bool aquad = at == PGA_SHAPE_QUAD, bquad = bt == PGA_SHAPE_QUAD;
-    if (aquad && !bquad) return sat_overlap(bm, bh, bh, am, ah, aq);
-    return sat_overlap(am, ah, aquad ? aq : ah, bm, bh, bquad ? bq : bh);
+    // one site for both orders: a wave that meets both kinds of collider would
+    // run two copies of the test one after the other
+    const bool swap = aquad && !bquad;
+    float A[12], Bm[12], af[3], ap[3], bf[3], bp[3];
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+        A[i] = swap ? bm[i] : am[i];
+        Bm[i] = swap ? am[i] : bm[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        af[i] = swap ? bh[i] : ah[i];
+        ap[i] = swap ? bh[i] : (aquad ? aq[i] : ah[i]);
+        bf[i] = swap ? ah[i] : bh[i];
+        bp[i] = swap ? aq[i] : (bquad ? bq[i] : bh[i]);
+    }
+    return sat_overlap(A, af, ap, Bm, bf, bp);
 }
 
 // Collider i of the store against the asking shape (bm, bs, shape): the tag
@@ -247,9 +262,8 @@ __device__ __forceinline__ bool shapes_overlap(const float am[12], const float a
 __device__ __forceinline__ bool collider_test(const float4* __restrict__ coll, uint32_t i, uint32_t tag,
                                               uint32_t phase, uint32_t shape, const float bm[12], const float bs[3]) {
     const float4* k = coll + 5u * i;
-    const float4 w3 = k[3], w4 = k[4];
+    const float4 w3 = k[3], w4 = k[4], w0 = k[0], w1 = k[1], w2 = k[2];   // one round trip
     if (__float_as_uint(w3.w) != tag || __float_as_uint(w4.y) >= phase) return false;
-    const float4 w0 = k[0], w1 = k[1], w2 = k[2];
     const float am[12] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
     const float as[3] = {w3.x, w3.y, w3.z};
     return shapes_overlap(am, as, __float_as_uint(w4.x), bm, bs, shape);
@@ -259,18 +273,21 @@ __device__ __forceinline__ bool collider_test(const float4* __restrict__ coll, u
 // stored with this tag overlap the shape? The store holds `n` such
 // colliders. With a BVH (built over them between phases, as
 // MultiPhaseEvaluator::execute does, GPUEvaluator.cuh:427-430) the walk of
-// BVHTraversal.cuh:21-148 runs without a stack over the nodes in
-// depth-first order: a node whose box meets the shape's box is entered (the
-// next node), any other skipped (its skip index); at a leaf the collider is
-// tested in full. The boxes are conservative, so the answer is the
-// existence over all n colliders, which a scan gives for few colliders.
+// BVHTraversal.cuh:21-148 visits the nodes whose box meets the shape's box and
+// tests the colliders it reaches in full. The boxes are conservative, so the
+// answer is the existence over all n colliders, which a scan gives for few
+// colliders.
+// The walk is a chain of dependent loads, at two waves per SIMD: its length is
+// what it costs. A node holds the boxes of four grandchildren, so that only
+// nodes whose own box was met are loaded, one 128-byte line for two binary
+// levels (1.2M props against 81,920 colliders: 408 us with 32-byte binary
+// nodes in depth-first order, where every rejected sibling is a load of its
+// own; 293 with these and the lanes' leaves tested together). A node that a
+// full stack could not take the children of is scanned, leaf by leaf.
 __device__ __forceinline__ bool collider_hit(const Ctx& c, uint32_t n, uint32_t tag, uint32_t phase,
-                                             uint32_t shape, float m0, float m1, float m2, float m3, float m4,
-                                             float m5, float m6, float m7, float m8, float m9, float m10, float m11,
-                                             float s0, float s1, float s2) {
-    const float bm[12] = {m0, m1, m2, m3, m4, m5, m6, m7, m8, m9, m10, m11};
-    const float bs[3] = {s0, s1, s2};
-    if (c.bvh_flat == nullptr || n <= 32u) {
+                                             uint32_t shape, const float bm[12], const float bs[3],
+                                             const CollMemo* memo) {
+    if (c.bvh_wide == nullptr || memo == nullptr || n <= 32u) {
 #pragma unroll 1
         for (uint32_t i = 0; i < n; ++i)
             if (collider_test(c.coll, i, tag, phase, shape, bm, bs)) return true;
@@ -278,18 +295,48 @@ __device__ __forceinline__ bool collider_hit(const Ctx& c, uint32_t n, uint32_t 
     }
     float lo[3], hi[3];
     shape_box(bm, bs, lo, hi);
-    const uint32_t nodes = 2u * n - 1u;
-    uint32_t i = 0;
+    uint32_t sp = 0, top = 0;            // the next node or leaf; those after it are on the stack
+    uint32_t p = 0, pe = 0;              // leaves left of a scanned node
+    auto pop = [&]() {
+        if (sp == 0u) return false;
+        --sp;
+        top = memo->stack[(sp >> 2) * memo->stride + (sp & 3u)];
+        return true;
+    };
+    bool more = true;
 #pragma unroll 1
-    while (i < nodes) {
-        const float4 w0 = c.bvh_flat[2u * i], w1 = c.bvh_flat[2u * i + 1u];
-        if (w0.x > hi[0] || w0.y > hi[1] || w0.z > hi[2] || w0.w < lo[0] || w1.x < lo[1] || w1.y < lo[2]) {
-            i = __float_as_uint(w1.z);          // skip the subtree
-            continue;
+    while (more) {
+        // every lane goes down to its next leaf before any lane tests one: a
+        // test is 250 instructions, and taken one lane at a time as each came
+        // to a leaf it ran once for most of the wave's steps
+#pragma unroll 1
+        while (more && p >= pe && !(top & kWideLeaf)) {   // no collider index has the bit: at most 2^26 of them
+            const float4* w = c.bvh_wide + 8u * top;
+            const float4 r = w[7];
+            if (sp + 4u > kWalkStack) {
+                p = __float_as_uint(r.x);
+                pe = __float_as_uint(r.y);
+                continue;
+            }
+            const float4 x0 = w[0], y0 = w[1], z0 = w[2], x1 = w[3], y1 = w[4], z1 = w[5], rf = w[6];
+            auto push = [&](float ax, float ay, float az, float bx, float by, float bz, float ref, uint32_t leaf_tag) {
+                bool miss = ax > hi[0] || ay > hi[1] || az > hi[2] || bx < lo[0] || by < lo[1] || bz < lo[2];
+                miss |= (__float_as_uint(ref) & kWideLeaf) != 0u && (leaf_tag & 0xFFFFu) != (tag & 0xFFFFu);
+                if (!miss && __float_as_uint(ref) != kWideNone) {
+                    memo->stack[(sp >> 2) * memo->stride + (sp & 3u)] = __float_as_uint(ref);
+                    ++sp;
+                }
+            };
+            push(x0.x, y0.x, z0.x, x1.x, y1.x, z1.x, rf.x, __float_as_uint(r.z));
+            push(x0.y, y0.y, z0.y, x1.y, y1.y, z1.y, rf.y, __float_as_uint(r.z) >> 16);
+            push(x0.z, y0.z, z0.z, x1.z, y1.z, z1.z, rf.z, __float_as_uint(r.w));
+            push(x0.w, y0.w, z0.w, x1.w, y1.w, z1.w, rf.w, __float_as_uint(r.w) >> 16);
+            more = pop();
         }
-        const uint32_t item = __float_as_uint(w1.w);
-        if (item != 0xFFFFFFFFu && collider_test(c.coll, item, tag, phase, shape, bm, bs)) return true;
-        ++i;
+        if (!more) break;
+        const uint32_t item = p < pe ? (uint32_t)c.bvh_keys[p++] : top & ~kWideLeaf;
+        if (collider_test(c.coll, item, tag, phase, shape, bm, bs)) return true;
+        if (p >= pe) more = pop();
     }
     return false;
 }
@@ -384,10 +431,7 @@ __device__ __forceinline__ int32_t apply_single(const Ctx& c, const E& e, Rec& r
             t = (memo->bits >> q) & 1u;         // the count pass's outcome
         } else {
             const uint32_t n = min(*c.coll_visible, c.coll_cap);
-            t = (n != 0u && collider_hit(c, n, f2u_rd(v0), rec_phase(c, r), e.shape(), r.m[0], r.m[1], r.m[2],
-                                         r.m[3], r.m[4], r.m[5], r.m[6], r.m[7], r.m[8], r.m[9], r.m[10], r.m[11],
-                                         r.s[0], r.s[1], r.s[2]))
-                    ? 0u : 1u;
+            t = (n != 0u && collider_hit(c, n, f2u_rd(v0), rec_phase(c, r), e.shape(), r.m, r.s, memo)) ? 0u : 1u;
             if (memo && memo->mode == 1u && q < 32u) memo->bits |= t << q;
         }
         if (memo) memo->n = q + 1u;
