@@ -199,7 +199,12 @@ __device__ __forceinline__ void run_level(const KArgs& a, LevelLDS& L, float4* P
                                           bool narrow) {
     const uint32_t nslots = a.prog.nslots, ncnt = nslots + 2u;
     const uint32_t w = wave_in_block();
-    const uint32_t wave = narrow ? w : (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    // neighbouring waves on neighbouring blocks: a level narrower than the grid
+    // spreads over all compute units, and a wider one ends evenly (16,384-lot
+    // city block 794 -> 761 us, a fit step of 256 lots 813 -> 786). With 16 or
+    // 32 children a wave in narrow levels, too, the city block's collider
+    // appends (one atomic a wave) took longer than the shorter walks saved.
+    const uint32_t wave = narrow ? w : w * gridDim.x + blockIdx.x;
     const uint32_t nwaves = (narrow ? blockDim.x : gridDim.x * blockDim.x) >> 6;
     stamp(a, level, 0);
     for (uint32_t k = lane_id(); k < ncnt; k += 64u) L.cnt[w][k] = 0u;
