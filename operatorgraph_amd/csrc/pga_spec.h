@@ -263,11 +263,13 @@ __device__ __forceinline__ void spec_pass(const KArgs& a, LevelLDS& L, float4* P
                             mode = back;
                             return;
                         }
-                        par_store(PW, cur);
+                        // a count pass needs the record again only for a leaf
+                        // fan-out's children: else most of it is never formed
+                        leaf = (e.flags() & EF_LEAF) != 0;
+                        if (WR || (leaf && !(e.flags() & EF_DIRECT))) par_store(PW, cur);
                         fe = e.idx;
                         fan_init(c, cur, e, f);
                         j = 0;
-                        leaf = (e.flags() & EF_LEAF) != 0;
                         start = !leaf;
                         const uint32_t sk = e.auxk(c, 0);
                         if (k == K_REPEAT) {
@@ -297,7 +299,7 @@ __device__ __forceinline__ void spec_pass(const KArgs& a, LevelLDS& L, float4* P
                             return;
                         }
                         // over-long chain: continues on the next level
-                        par_store(PW, cur);
+                        if (WR) par_store(PW, cur);
                         fe = e.idx;
                         self = true;
                         f.n = 1;
