@@ -375,7 +375,14 @@ __device__ __noinline__ float exp_eval(const WordT* __restrict__ b, float m0, fl
     return top == 1 ? st0 : top == 2 ? st1 : top == 3 ? st2 : st3;
 }
 
-__device__ __noinline__ float philox_uniform(uint32_t axiom, uint32_t path, uint32_t depth, uint32_t stream,
+// inline in a specialised kernel, which has few sites (the stochastic batch
+// 340 -> 332 us), a call in the interpreting ones, which have one per operator
+#ifdef __HIPCC_RTC__
+__device__ __forceinline__
+#else
+__device__ __noinline__
+#endif
+float philox_uniform(uint32_t axiom, uint32_t path, uint32_t depth, uint32_t stream,
                                              uint32_t k0, uint32_t k1) {
     uint32_t u = philox_x0(axiom, path, depth, stream, k0, k1);
     return (float)(u >> 8) * 5.9604644775390625e-8f;   // top 24 bits, exact
