@@ -39,16 +39,21 @@ __device__ __forceinline__ void adj_zero(Adj& d) {
 
 // dL/dparams of one thread. A thread replays one child, so every
 // contribution is to the same axiom: up to kGradSlots per-axiom parameters
-// accumulate in registers (FP64) and leave once, at the end (flush_grads).
+// accumulate in FP64 and leave once, at the end (flush_grads). The sums are in
+// LDS, parameter q of the wave's lane l at word q * 64 + l of the wave's 4 KB:
+// one LDS addition a contribution, where sums in registers, whose index must
+// be a constant, took eight selected FP64 additions and 16 registers.
 constexpr uint32_t kGradSlots = 8;
+typedef __attribute__((address_space(3))) double lds_f64;
 struct GradAcc {
-    double v[kGradSlots];
+    lds_f64* v;       // the lane's: parameter q at v[q * 64]
     uint32_t axiom;   // ~0u: no contribution yet
 };
 
-__device__ __forceinline__ void grad_zero(GradAcc& ga) {
+__device__ __forceinline__ void grad_zero(GradAcc& ga, lds_f64* wave) {
+    ga.v = wave + (threadIdx.x & 63u);
 #pragma unroll
-    for (uint32_t q = 0; q < kGradSlots; ++q) ga.v[q] = 0.0;
+    for (uint32_t q = 0; q < kGradSlots; ++q) ga.v[q * 64u] = 0.0;
     ga.axiom = ~0u;
 }
 
@@ -63,36 +68,54 @@ __device__ __forceinline__ void grad_param(const Ctx& c, const AdjArgs& g, GradA
     const uint32_t slot = (uint32_t)p.a;
     if (c.aparams_per <= kGradSlots && slot < kGradSlots && (ga.axiom == ~0u || ga.axiom == axiom)) {
         ga.axiom = axiom;
-#pragma unroll
-        for (uint32_t q = 0; q < kGradSlots; ++q) ga.v[q] += q == slot ? (double)v : 0.0;
+        // the lane's own word: an atomic for its form, one instruction and no wait
+        __hip_atomic_fetch_add(ga.v + slot * 64u, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     } else {
         atomicAdd(g.grad + (size_t)axiom * c.aparams_per + slot, (double)v);
     }
 }
 
-// The accumulated contributions to the FP64 gradient: a full wave whose
-// contributions all go to one axiom sums each parameter across its lanes
-// first (one atomic per parameter instead of one per lane and operator);
-// other waves add lane by lane.
+// The wave's contributions to the FP64 gradient, axiom by axiom: the lanes of
+// one axiom are summed first, and every parameter of it is one global atomic.
+// Eight lanes take a parameter each, so that all are summed at once: eight
+// LDS reads (no two of the eight groups on the same chunk of lanes, against
+// bank conflicts) and three shuffles, where a parameter after the other went
+// through six shuffles of the whole wave. Fewer than eight lanes of an axiom
+// add for themselves, which measures what reducing from two lanes on does; the
+// atomics of many lanes on one line are what costs (reducing from 24 lanes on:
+// 609 us instead of 434 for the second level from the end of 4,096 lots, 94
+// instead of 32 for 256 lots). Every lane of the wave calls it.
 __device__ __forceinline__ void flush_grads(const Ctx& c, const AdjArgs& g, const GradAcc& ga) {
     const uint32_t per = c.aparams_per;
     if (per == 0u || per > kGradSlots) return;
-    const bool has = ga.axiom != ~0u;
-    const unsigned long long act = __ballot(1), hm = __ballot(has);
-    if (hm == 0ull) return;
-    const int lead = __ffsll((long long)hm) - 1;
-    const uint32_t ax0 = __shfl(ga.axiom, lead);
-    const bool uniform = act == ~0ull && __ballot(has && ga.axiom != ax0) == 0ull;
+    unsigned long long left = __ballot(ga.axiom != ~0u);
+    if (left == 0ull) return;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t lane = threadIdx.x & 63u, q = lane >> 3;
+    const lds_f64* wave = ga.v - lane;
+#pragma unroll 1
+    while (left != 0ull) {
+        const uint32_t ax = (uint32_t)__builtin_amdgcn_readlane((int)ga.axiom, __ffsll((long long)left) - 1);
+        const unsigned long long of = __ballot(ga.axiom == ax);
+        left &= ~of;
+        if (__popcll(of) >= 8) {
+            double x = 0.0;
 #pragma unroll
-    for (uint32_t q = 0; q < kGradSlots; ++q) {   // unrolled: ga.v stays in registers
-        if (q >= per || __ballot(ga.v[q] != 0.0) == 0ull) continue;
-        if (uniform) {
-            double x = ga.v[q];
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const uint32_t l = (lane & 7u) + 8u * ((k + q) & 7u);
+                const double w = wave[q * 64u + l];
+                x += (of >> l) & 1ull ? w : 0.0;
+            }
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) x += __shfl_xor(x, d);
-            if ((int)(threadIdx.x & 63u) == lead) atomicAdd(g.grad + (size_t)ax0 * per + q, x);
-        } else if (ga.v[q] != 0.0) {
-            atomicAdd(g.grad + (size_t)ga.axiom * per + q, ga.v[q]);
+            for (int d = 4; d >= 1; d >>= 1) x += __shfl_xor(x, d);
+            if ((lane & 7u) == 0u && q < per && x != 0.0) atomicAdd(g.grad + (size_t)ax * per + q, x);
+        } else if (ga.axiom == ax) {
+            for (uint32_t k = 0; k < per; ++k) {
+                const double w = ga.v[k * 64u];
+                if (w != 0.0) atomicAdd(g.grad + (size_t)ax * per + k, w);
+            }
         }
     }
 }
@@ -548,10 +571,11 @@ __device__ __forceinline__ void child_start(const KArgs& a, const AdjArgs& g, co
 // stored lane by lane, 312 MB of them became 716 MB of writes. The levels of
 // 4,096 parameterised lots, last first: 372 / 661 / 295 / 67 us with 80-byte
 // slots, the program read from memory and 48 bytes of scratch a lane; 299 /
-// 559 / 227 / 52 like this.
+// 559 / 227 / 52 us with that; 297 / 434 / 190 / 60 with the gradient sums in
+// LDS too.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_adjoint(KArgs a, AdjArgs g) {
     __shared__ AdjLDS T;
-    __shared__ float4 stage[4][256];     // per wave: 64 slots on their way out
+    __shared__ float4 stage[4][256];     // per wave: the gradient sums, then 64 slots on their way out
     adj_stage(a, g, T);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const Ctx c = adj_ctx(a, T);
@@ -572,7 +596,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     Adj d;
     adj_zero(d);
     GradAcc ga;
-    grad_zero(ga);
+    grad_zero(ga, (lds_f64*)stage[threadIdx.x >> 6]);
     if (kind != T_DROP) {
         // replay the chain of single-child operators to its end
         uint32_t steps = 0;
@@ -613,6 +637,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     }
     flush_grads(c, g, ga);
     if (g.level == 0u) return;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");      // the sums are read: the words are the slots'
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     Adj dp;
     float d_o = 0.0f, d_ns = 0.0f;
     const uint32_t axis = ch.dv.y >> 30;
