@@ -354,6 +354,7 @@ __device__ __forceinline__ void fan_adj(const Ctx& c, const AdjArgs& g, GradAcc&
     // parent-state adjoints the children left (four 16-byte loads per slot),
     // and the sum of their offset adjoints in child order
     float total_o = 0.0f;
+#pragma unroll 2                       // two children's loads in flight: 434 -> 417 us (see k_adjoint)
     for (uint32_t q = 0; q < nd; ++q) {
         const float4* sl = slot_at(g, first + q);
         float4 a = sl[0], b = sl[1], cc = sl[2], dd = sl[3];
@@ -572,8 +573,11 @@ __device__ __forceinline__ void child_start(const KArgs& a, const AdjArgs& g, co
 // 4,096 parameterised lots, last first: 372 / 661 / 295 / 67 us with 80-byte
 // slots, the program read from memory and 48 bytes of scratch a lane; 299 /
 // 559 / 227 / 52 us with that; 297 / 434 / 190 / 60 with the gradient sums in
-// LDS too.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_adjoint(KArgs a, AdjArgs g) {
+// LDS too, and 285 / 389 / 187 / 62 with four waves per SIMD instead of three,
+// which the registers that these sums took now allow (64 bytes of scratch a
+// lane instead of 32: 256 lots, a third of a round of the grid, lose 3 of 125
+// us by it), and the loads of two children's slots in flight.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_adjoint(KArgs a, AdjArgs g) {
     __shared__ AdjLDS T;
     __shared__ float4 stage[4][256];     // per wave: the gradient sums, then 64 slots on their way out
     adj_stage(a, g, T);
