@@ -82,6 +82,21 @@ def test_collision_pairs(E, quad_depth):
     assert 0.2 * len(kinds) < len(got[1]) < 0.8 * len(kinds)
 
 
+@pytest.mark.parametrize("pairs", [32, 33, 65, 9001])
+def test_collision_walk_of_overlapping_colliders(E, pairs):
+    """Colliders that lie on each other, on either side of the count that is
+    scanned and with more of them than a walk's stack can hold the subtrees
+    of; every other question asks for a tag that differs from its collider's
+    in the bits above the low 16 only, and no shape meets it."""
+    _note(f"collision walk pairs={pairs}")
+    rng = np.random.default_rng(29)
+    ax, p = axioms.collision_pair_axioms([(B, B)] * pairs, rng, spread=0.3)
+    p[1::4, 9] += 65536.0
+    got, ref, phases = check(E, grammars.collision_pairs(), ax, 3, params=p)
+    assert phases == 2 and len(got[0]) == pairs
+    assert len(got[1]) <= pairs // 2 and len(got[2]) >= (pairs + 1) // 2
+
+
 @pytest.mark.parametrize("technique", TECHNIQUES)
 @pytest.mark.parametrize("walls", [False, True])
 def test_context_city(E, technique, walls):

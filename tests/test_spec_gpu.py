@@ -90,6 +90,27 @@ def test_spec_every_operator(block_size):
         spec_check(_compsplit_program(parallel), _boxes(50, 17), 3, block_size=block_size)
 
 
+@pytest.mark.parametrize("children", [1, 2, 7, 8, 9, 16])
+def test_spec_leaf_fans(children):
+    """Fan-outs of terminals and Discards alone, on either side of the width
+    up to which their rounds are unrolled, the last wave one lane full: two
+    terminals taken in turn, every fifth child dropped."""
+    _note(f"specialised: leaf fan-out of {children} children")
+    from operatorgraph_amd.program import DispatchTable, Entry, Program, Scalar
+    WALL, WINDOW, NONE = 1, 2, 3
+    succ = [NONE if j % 5 == 4 else (WALL, WINDOW)[j % 2] for j in range(children)]
+    weights = [-1.0 - 0.25 * j for j in range(children)]
+    table = DispatchTable([
+        grammars.subdiv_entry(B, abi.X, weights, succ),
+        Entry(grammars.op(abi.GENERATE, B, 1), [Scalar(0)], []),
+        Entry(grammars.op(abi.GENERATE, B, 1), [Scalar(1)], []),
+        Entry(grammars.op(abi.DISCARD, B), [], []),
+    ])
+    for n in (1, 65):
+        got, _ = spec_check(Program(grammars.INTERPRETER_PROCEDURES, table, f"fan{children}"), _boxes(n, 23), 2)
+        assert [len(g) for g in got] == [n * succ.count(WALL), n * succ.count(WINDOW)]
+
+
 @pytest.mark.parametrize("name", sorted(k for k, v in grammar_fixture().items() if "refused" not in v))
 def test_spec_reference_grammar(name):
     _note(f"specialised: reference grammar {name}")
