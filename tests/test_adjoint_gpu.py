@@ -359,6 +359,31 @@ def test_adjoint_wave_edges_vs_fp64(n):
     _assert_close(grad, ref)
 
 
+@pytest.mark.parametrize("children", [1, 2, 7, 8, 9, 33])
+def test_adjoint_axioms_sharing_a_wave(children):
+    """A wave with the children of several axioms sums the parameters axiom by
+    axiom, from eight children of one on: Repeat(X, 1) Translate(p0, p1, 0)
+    Scale(p2, -1, -1) Generate(0) over `children` tiles each. FP32 terms of
+    both signs: their rounding against the largest parameter of the axiom."""
+    _note(f"adjoint of {children} children an axiom")
+    table = DispatchTable([
+        Entry(op(abi.REPEAT, Q), [Scalar(abi.X), Scalar(1.0), Scalar(abi.ADJUST_TO_FILL)], [(1, 0)]),
+        Entry(op(abi.TRANSLATE, Q), [AxiomParam(0), AxiomParam(1), Scalar(0.0)], [(2, 0)]),
+        Entry(op(abi.SCALE, Q), [AxiomParam(2), Scalar(-1.0), Scalar(-1.0)], [(3, 0)]),
+        Entry(op(abi.GENERATE, Q, 1), [Scalar(0)], []),
+    ])
+    n = 37
+    rng = np.random.default_rng(children)
+    ax = axioms.empty(n)
+    ax["size"] = np.stack([np.full(n, children + 0.25), rng.uniform(1, 2, n), np.zeros(n)], axis=1)
+    ax["model"][:, [3, 7, 11]] = rng.uniform(-5, 5, size=(n, 3)).astype(np.float32)
+    ax["shape_type"] = Q
+    params = rng.uniform(0.2, 0.8, size=(n, 3)).astype(np.float32)
+    grad, ref, r = _adjoint_pair(Program(grammars.INTERPRETER_PROCEDURES, table, "tiles"), ax, params, 1)
+    assert r.count(0) == n * children
+    _assert_close(grad, ref, rel=1e-4, entry_rel=5e-2)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 513, 512 * 512 - 1, 512 * 512 + 65])
 def test_fused_loss_tile_edges(n):
     """The fused loss at the edges of a wave's tile, a workgroup and the
