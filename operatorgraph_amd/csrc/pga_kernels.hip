@@ -19,10 +19,12 @@
 // accumulates per-wave totals in LDS (terminals per terminal slot, parents,
 // descriptors), blocks publish their totals, a grid barrier, each block
 // scans the totals of the blocks before it, and a write pass recomputes the
-// children and writes at exact offsets. Same-address global atomics sustain
-// only ~1e8/s on this device, so per-wave atomics would bound the kernel;
-// the scan also makes the output order deterministic. The count pass skips
-// model-matrix arithmetic when no decision of the program reads the matrix.
+// children and writes at exact offsets. A level that one block's threads hold
+// is run by block 0 alone, without the grid's barriers. Same-address global
+// atomics sustain only ~1e8/s on this device, so per-wave atomics would bound
+// the kernel; the scan also makes the output order deterministic. The count
+// pass skips model-matrix arithmetic when no decision of the program reads the
+// matrix.
 //
 // Two techniques share that level body:
 //   k_level  - one cooperative launch per level, the host reads the next
