@@ -459,7 +459,10 @@ PGA_API pga_status pga_lbvh_seconds(pga_lbvh* bvh, double* seconds);
  * enqueued on `stream` (a hipStream_t of the current device; NULL: the
  * default stream) and the call returns without waiting. Calls that overlap
  * on one GPU share the array and race: order them on one stream or wait in
- * between. Outputs as pga_lbvh_build. */
+ * between. Builds that overlap all the same leave undefined values in their
+ * outputs and can take some 100 ms longer (they wait for sort tiles that the
+ * other build has cleared), but they end and stay inside their own arrays.
+ * Outputs as pga_lbvh_build. */
 #define PGA_LBVH_NOALLOC_MAX_LEAVES (1u << 20)
 PGA_API pga_status pga_lbvh_build_noalloc(const float* aabbs, uint32_t n, const float scene_min[3],
                                           const float scene_max[3], uint64_t* keys, int32_t* left, int32_t* right,

@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libpga_amd.so")
 SOURCES = ["pga_kernels.hip", "pga_adjoint.hip", "pga_lbvh.hip", "pga_loss.hip", "pga_mesh.hip", "pga_api.cpp",
            "pga_spec.cpp"]
 HOST_SOURCES = ["pga_compiler.cpp"]   # no device code: built with the host compiler
-HEADERS = ["pga_device.h", "pga_ops.h", "pga_kernels.h", "pga_level.h", "pga_spec.h", "pga_spec_host.h"]
+HEADERS = ["pga_device.h", "pga_ops.h", "pga_kernels.h", "pga_level.h", "pga_spec.h", "pga_spec_host.h", "pga_lookback.h"]
 # device headers compiled again at run time (hipRTC) for the kernels
 # specialised to one program; embedded in the library as text
 RTC_HEADERS = [("pga.h", os.path.join(ROOT, "include", "pga.h"))] + \

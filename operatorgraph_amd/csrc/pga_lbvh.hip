@@ -40,6 +40,7 @@
 #include <string>
 
 #include "../../include/pga.h"
+#include "pga_lookback.h"
 
 namespace bvhk {
 
@@ -54,7 +55,6 @@ constexpr uint32_t kGatherBlocks = 8192;         // grid-stride workgroups of th
 constexpr uint32_t kTreeTile = 1024;             // sorted leaves per workgroup of the tree's first level
 constexpr uint32_t kTreeGroup = 32;              // workgroups of one level whose open subtrees one of the next takes
 constexpr uint32_t kMaxRoots = 128;              // open subtrees a workgroup may leave (see k_tree_leaves)
-typedef unsigned long long u64;
 // two floats of a box record: boxes are 24-byte records that a caller may align to 4 bytes only
 typedef float box2 __attribute__((ext_vector_type(2), aligned(4)));
 
@@ -350,21 +350,18 @@ __device__ __forceinline__ uint32_t rank_tile(SortLDS& S, const u64 key[kItems],
     return total;
 }
 
-// Status words of the look-back: the tile's count of a digit (kCount), or
-// with all tiles before it (kPrefix), in the low 62 bits. One 64-bit word
-// carries flag and value, so relaxed agent-scope accesses order themselves.
-constexpr u64 kCount = 1ull << 62, kPrefix = 2ull << 62, kValue = (1ull << 62) - 1ull;
+// Idle looks of the look-back before it counts a tile's digit itself: 10 to 20
+// ms, a thousand times what a word takes to come.
+constexpr uint32_t kPatience = 1u << 14;
 
 // One pass: the tile's keys ranked in LDS, the tile's place in the output of
 // every digit found by looking back over the tiles before it, the keys
 // written in tile order (runs of consecutive keys per digit). A tile waits
 // for lower tiles only, and tiles are numbered by ticket in the order in
 // which workgroups start, so the lowest unfinished tile is always running and
-// never waits: every wait ends. The look-back reads eight tiles at a time:
-// their words are independent loads, and one at a time the tiles of a million
-// keys would be a chain of up to 245 round trips to memory. A million keys
-// sort in 4 x 16.7 us; a histogram, three scan launches and a scatter a pass
-// took 181 us (20 launches).
+// never waits; and no wait is longer than kPatience looks (look_back). A
+// million keys sort in 4 x 16.7 us; a histogram, three scan launches and a
+// scatter a pass took 181 us (20 launches).
 __global__ void __launch_bounds__(kThreads) k_sweep(const u64* __restrict__ in, u64* __restrict__ out, uint32_t n,
                                                     const uint32_t* nd, uint32_t pass,
                                                     const uint32_t* __restrict__ totals, u64* status,
@@ -394,25 +391,18 @@ __global__ void __launch_bounds__(kThreads) k_sweep(const u64* __restrict__ in, 
         if (w * 256u + it * 64u + lane < cnt) S.key[rank[it]] = key[it];
     const uint32_t g = scan256(t < kDigits ? totals[pass * kDigits + t] : 0u, S.sums);
     if (t < kDigits) {
-        uint32_t before = 0;
-        int64_t k = (int64_t)tile - 1;                  // the nearest tile not yet added
-        constexpr int kBack = 8;
-        while (k >= 0) {
-            u64 v[kBack];
-#pragma unroll
-            for (int b = 0; b < kBack; ++b)
-                v[b] = __hip_atomic_load(&st[(size_t)(k - b > 0 ? k - b : 0) * kDigits], __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-            bool open = true;                           // every nearer word has been there
-#pragma unroll
-            for (int b = 0; b < kBack; ++b) {
-                if (!open || k < 0) continue;
-                if (v[b] < kCount) { open = false; continue; }
-                before += (uint32_t)(v[b] & kValue);
-                k = v[b] >= kPrefix ? -1 : k - 1;
-            }
-            if (!open) __builtin_amdgcn_s_sleep(1);
-        }
+        const uint32_t before = look_back(
+            tile, kPatience,
+            [&](uint32_t k) {
+                return __hip_atomic_load(&st[(size_t)k * kDigits], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            },
+            [] { __builtin_amdgcn_s_sleep(1); },
+            [&](uint32_t k) {                           // tile k < tile: all its keys are there
+                uint32_t c = 0;
+#pragma unroll 8
+                for (uint32_t q = 0; q < kTile; ++q) c += ((uint32_t)(in[(size_t)k * kTile + q] >> shift) & 0xFFu) == t;
+                return c;
+            });
         if (tile)
             __hip_atomic_store(&st[(size_t)tile * kDigits], kPrefix | (u64)(before + total), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
@@ -425,7 +415,7 @@ __global__ void __launch_bounds__(kThreads) k_sweep(const u64* __restrict__ in, 
         if (q < cnt) {
             const u64 x = S.key[q];
             const uint32_t off = S.base[(uint32_t)(x >> shift) & 0xFFu] + q;
-            if (off < n) out[off] = x;                  // always true: the totals count these keys
+            if (off < n) out[off] = x;                  // always true for a build that has its scratch to itself
         }
     }
 }
@@ -538,8 +528,8 @@ __device__ __forceinline__ int key_delta(const u64* __restrict__ keys, uint32_t 
 // through global memory (three kernels, which read the topology back) took
 // 142 us for what the levels here do in 45 + 46.
 template <bool LEAVES, uint32_t CAP>
-__device__ __forceinline__ void climb(TreeLDS<CAP>& T, LeafOut* lo, const RootIn* in, const TreeOut& out, uint32_t m,
-                                      uint32_t q, float2 b0, float2 b1, float2 b2) {
+__device__ __forceinline__ void climb(TreeLDS<CAP>& T, LeafOut* lo, const RootIn* in, const TreeOut& out, uint32_t n,
+                                      uint32_t m, uint32_t q, float2 b0, float2 b1, float2 b2) {
     uint32_t ql = q, qr = q;
     uint32_t L = LEAVES ? q : in->first[q], R1 = LEAVES ? q + 1u : in->first[q + 1u];   // leaves [L, R1)
     int dl = T.delta[ql], dr = T.delta[qr + 1u];
@@ -557,7 +547,9 @@ __device__ __forceinline__ void climb(TreeLDS<CAP>& T, LeafOut* lo, const RootIn
                 pl[P - 1u] = (uint16_t)node;
                 pr[P] = (uint16_t)node;
                 lo->other_end[node] = (uint16_t)(node == L ? R1 - 1u : L);
-            } else {
+            } else if (node < n - 1u && P - 1u < n - 1u && (rleaf || P < n - 1u)) {
+                // (always; the open subtrees come from memory that a build which
+                // breaks the rule of pga_lbvh_build_noalloc writes, too)
                 const int32_t lc = lleaf ? (int32_t)(P - 1u) : -(int32_t)(P - 1u), rc = rleaf ? (int32_t)P : -(int32_t)P;
                 out.left[node] = lc;
                 out.right[node] = rc;
@@ -690,7 +682,7 @@ __global__ void __launch_bounds__(kThreads) k_tree_leaves(const float* __restric
     const uint32_t m = min(kTreeTile, n - s);
     const uint32_t i = s + min(q, m - 1u);
     const u64 key = keys[i];
-    const box2* src = reinterpret_cast<const box2*>(aabbs + (size_t)(uint32_t)key * 6u);
+    const box2* src = reinterpret_cast<const box2*>(aabbs + (size_t)min((uint32_t)key, n - 1u) * 6u);
     const box2 g0 = src[0], g1 = src[1], g2 = src[2];
     T.slot[q] = 0u;
     T.mark[q] = 0u;
@@ -699,7 +691,7 @@ __global__ void __launch_bounds__(kThreads) k_tree_leaves(const float* __restric
     if (q == 0u) T.delta[m] = (int8_t)key_delta(keys, s + m, n);
     __syncthreads();
     if (q < m)
-        climb<true>(T, &O, nullptr, out, m, q, make_float2(g0.x, g0.y), make_float2(g1.x, g1.y),
+        climb<true>(T, &O, nullptr, out, n, m, q, make_float2(g0.x, g0.y), make_float2(g1.x, g1.y),
                     make_float2(g2.x, g2.y));
     leave_roots(T, nullptr, s, m, roots + (size_t)blockIdx.x * kMaxRoots, nroots + blockIdx.x);
     if (q >= m) return;
@@ -765,7 +757,7 @@ __global__ void __launch_bounds__(kThreads) k_tree_roots(const u64* __restrict__
     }
     __syncthreads();
     for (uint32_t q = t; q < m; q += kThreads)
-        climb<false>(T, nullptr, &I, out, m, q, T.box[q * 3u], T.box[q * 3u + 1u], T.box[q * 3u + 2u]);
+        climb<false>(T, nullptr, &I, out, n, m, q, T.box[q * 3u], T.box[q * 3u + 1u], T.box[q * 3u + 2u]);
     leave_roots(T, &I, 0u, m, roots + (size_t)blockIdx.x * kMaxRoots, nroots + blockIdx.x);
 }
 
