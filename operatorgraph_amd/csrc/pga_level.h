@@ -534,8 +534,10 @@ __device__ __forceinline__ void scan_counts(const KArgs& a, LevelLDS& L, uint32_
     // the totals are all that crosses this barrier: written and read at agent
     // scope, complete before the block arrives. With the fences of
     // grid_barrier a scan took 5.5 us at 256 workgroups, and the write pass
-    // read the children the count pass had just read from memory again
-    __builtin_amdgcn_s_waitcnt(0);
+    // read the children the count pass had just read from memory again. The
+    // wait clobbers memory, so that the compiler keeps the stores before it
+    // (the builtin of the instruction does not touch memory for it)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     grid_barrier<false>(a.bar, gridDim.x, L.gen);
     // wave w sums counters k = w, w + nw, ... over the blocks, 64 blocks a step
     for (uint32_t k = wave_in_block(); k < ncnt; k += nw) {
