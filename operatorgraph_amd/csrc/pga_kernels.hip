@@ -39,7 +39,12 @@ namespace pga {
 
 // One pass over the children of a level; waves take 64 consecutive
 // children at a time, in a fixed order, so both passes see the same lanes.
-template <bool TAPE, bool CS>
+// AHEAD: the next children's descriptors are read an iteration ahead and stay
+// in registers through the state machine. Builds of up to 512 threads have
+// registers for that (16,384 lots at 512: 982 -> 961 us); larger ones spill,
+// inside the machine's loop (the same lots at 1,024: 1,112 us without, 1,669
+// with; at 768 it makes no difference: 796 and 796).
+template <bool TAPE, bool CS, bool AHEAD>
 __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS& L, float4* PW, bool wr,
                                          uint32_t level, uint32_t n, uint32_t wave, uint32_t nwaves) {
     // inputs: written by level - 1 (ping-pong buffers, or that level's part of the tape)
@@ -47,12 +52,13 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
     const Desc* desc_in = TAPE ? a.tape_desc + L.td_prev : ((level & 1u) ? a.desc0 : a.desc1);
     const uint32_t child_base = level == 0u ? 0u : a.n_axioms + L.td_prev;   // tape outcomes
     f4* ST = reinterpret_cast<f4*>(PW + 5u * blockDim.x) + wave_in_block() * 256u;
-    uint4 dnext = load_desc(desc_in, level, wave * 64u + lane_id(), n);
+    uint4 dnext = {};
+    if (AHEAD) dnext = load_desc(desc_in, level, wave * 64u + lane_id(), n);
 #pragma unroll 1
     for (uint32_t base = wave * 64u; base < n; base += nwaves * 64u) {
         const uint32_t i = base + lane_id();
-        const uint4 dv = dnext;
-        dnext = load_desc(desc_in, level, i + nwaves * 64u, n);    // n < 2^31: no wrap
+        const uint4 dv = AHEAD ? dnext : load_desc(desc_in, level, i, n);
+        if (AHEAD) dnext = load_desc(desc_in, level, i + nwaves * 64u, n);    // n < 2^31: no wrap
         Rec cur;
         bool valid = i < n && load_child(a, c, par_in, dv, wr, level, i, cur);
         // an axiom whose entry reaches no phase of this launch adds nothing
@@ -196,7 +202,7 @@ __device__ __forceinline__ void run_pass(const KArgs& a, const Ctx& c, LevelLDS&
 // One derivation level: count pass, scan, write pass. Leaves L.next_n =
 // children of the next level; block 0 records the level's parent and
 // descriptor counts. narrow: this block runs the level alone.
-template <bool TAPE, bool CS>
+template <int BS, bool TAPE, bool CS>
 __device__ __forceinline__ void run_level(const KArgs& a, LevelLDS& L, float4* PW, uint32_t level, uint32_t n,
                                           bool narrow) {
     const uint32_t nslots = a.prog.nslots, ncnt = nslots + 2u;
@@ -214,7 +220,7 @@ __device__ __forceinline__ void run_level(const KArgs& a, LevelLDS& L, float4* P
     for (uint32_t pass = 0; pass < 2u; ++pass) {
         const bool wr = pass != 0u;
         const Ctx c = make_ctx<TAPE, CS>(a, L, level, wr);
-        run_pass<TAPE, CS>(a, c, L, PW, wr, level, n, wave, nwaves);
+        run_pass<TAPE, CS, (BS <= 512)>(a, c, L, PW, wr, level, n, wave, nwaves);
         __syncthreads();
         if (!wr && narrow) scan_block(a, L, level);
         else if (!wr) scan_counts(a, L, level, level);
@@ -238,7 +244,7 @@ __global__ void __launch_bounds__(BS) k_level(KArgs a, uint32_t level) {
     init_barrier(a, L);
     init_bases(a, L);
     const uint32_t n = first_level_size(a, level);
-    if (n != 0u) run_level<false, CS>(a, L, PW, level, n, false);
+    if (n != 0u) run_level<BS, false, CS>(a, L, PW, level, n, false);
     // every block has read the old bases before the barrier inside run_level
     store_bases(a, L);
 }
@@ -286,7 +292,7 @@ __global__ void __launch_bounds__(BS) k_mega(KArgs a) {
     while (level < a.max_levels && n != 0u) {
         const bool narrow = n <= BS;
         if (!narrow || blockIdx.x == 0) {
-            run_level<TAPE, CS>(a, L, PW, level, n, narrow);
+            run_level<BS, TAPE, CS>(a, L, PW, level, n, narrow);
             n = next_level<TAPE>(a, L);
             ++level;
             if (narrow) {

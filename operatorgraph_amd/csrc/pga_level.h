@@ -436,9 +436,10 @@ __device__ __forceinline__ bool load_axiom(const KArgs& a, const Ctx& c, uint32_
     return true;
 }
 
-// The descriptor of child i (level 0 has none). The passes read it an
-// iteration ahead: the parent it names is one more dependent load, and at two
-// or three waves per SIMD the two round trips were most of a count pass.
+// The descriptor of child i (level 0 has none). A pass with registers to hold
+// it reads it an iteration ahead: the parent it names is one more dependent
+// load, and at two or three waves per SIMD the two round trips were most of a
+// count pass.
 __device__ __forceinline__ uint4 load_desc(const Desc* desc_in, uint32_t level, uint32_t i, uint32_t n) {
     return level != 0u && i < n ? *reinterpret_cast<const uint4*>(desc_in + i) : make_uint4(0u, kDescNone, 0u, 0u);
 }

@@ -156,6 +156,32 @@ def test_kitchen_sink_operators(E, technique):
     assert sum(len(g) for g in got) > 64
 
 
+@pytest.mark.parametrize("technique", TECHNIQUES)
+def test_largest_workgroups_keep_up(E, technique):
+    """1,024 threads leave half the registers that 512 do, and a value held
+    across the state machine is spilled there: 16,384 lots took 1.75 times the
+    512-thread build's time with one such value and 1.16 times without. The
+    bound lies between."""
+    _note(f"workgroups of 1024 against 512 threads, technique={technique}")
+    lots = axioms.facade_lots(16384)
+    walls, windows = axioms.facade_lot_terminals(lots)
+    best = {}
+    for bs in (512, 1024):
+        eng = E.Engine(technique=technique, block_size=bs, queue_capacity=1 << 23)
+        try:
+            eng.load(grammars.facade()).set_axioms(lots)
+            eng.bind(0, int(walls.sum()))
+            eng.bind(1, int(windows.sum()))
+            times = []
+            for _ in range(10):
+                eng.execute()
+                times.append(eng.kernel_seconds())
+            best[bs] = min(times)
+        finally:
+            eng.close()
+    assert best[1024] < 1.45 * best[512], best
+
+
 @pytest.mark.parametrize("block_size", [256, 768, 1024])
 def test_workgroup_size_variants(E, block_size):
     # each workgroup size is its own kernel build (register budget 256/168/128)
