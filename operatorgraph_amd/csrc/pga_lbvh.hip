@@ -764,6 +764,14 @@ __global__ void __launch_bounds__(kThreads) k_tree_roots(const u64* __restrict__
 // The tree with four children a node, for walks (collider_hit): binary node i
 // takes its children's children, or a child itself where it is a leaf. One
 // thread per binary node (a walk from the root meets those at even depths).
+// A child of more than a third of the node's leaves stands first: a walk
+// pushes the children in this order and goes on with the last, so that it is
+// in such a child only when no sibling of it waits on the stack. With 17 words
+// waiting (no room for four more), at least six levels have some, and the walk
+// is in at most 3^-6 = 1/729 of the leaves. Nodes of up to 32 leaves, which
+// are quickly scanned, keep the order of the curve: it finds a collision
+// sooner (16,384-lot city block 764 us, 766 with this rule, 773 with it for
+// all nodes, 769 with all four children sorted by size).
 __global__ void __launch_bounds__(256) k_wide(const u64* __restrict__ keys, uint32_t n, const uint32_t* nd,
                                               const int32_t* __restrict__ left, const int32_t* __restrict__ right,
                                               const int32_t* __restrict__ other_end,
@@ -772,45 +780,62 @@ __global__ void __launch_bounds__(256) k_wide(const u64* __restrict__ keys, uint
     const uint32_t nn = leaf_count(n, nd);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (nn < 2u || i >= nn - 1u) return;
-    float b[4][6];
-    uint32_t ref[4], tag[4];
+    // a left child of [l, r] ends, and a right child begins, at the split
+    const uint32_t far = (uint32_t)other_end[i], l = min(i, far), r = max(i, far);
+    int32_t g[4];                        // the slots' subtrees
+    uint32_t size[4];                    // their leaves, 0: no subtree
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int32_t c = h == 0 ? left[i] : right[i];
-        int32_t g[2] = {c, 0};           // the slots' subtrees
-        bool two = false;
-        if (c < 0) {
-            g[0] = left[-c];
-            g[1] = right[-c];
-            two = true;
+        const uint32_t at = (uint32_t)abs(c), first = h == 0 ? l : at, last = h == 0 ? at : r;
+        g[2 * h] = c < 0 ? left[at] : c;
+        g[2 * h + 1] = c < 0 ? right[at] : 0;
+        size[2 * h] = c < 0 ? (uint32_t)abs(g[2 * h]) - first + 1u : 1u;
+        size[2 * h + 1] = c < 0 ? last - (uint32_t)abs(g[2 * h + 1]) + 1u : 0u;
+    }
+    uint32_t big = 0, most = size[0];
+#pragma unroll
+    for (uint32_t q = 1; q < 4u; ++q) {
+        big = size[q] > most ? q : big;
+        most = max(most, size[q]);
+    }
+    if (r - l < 32u || most <= (r - l + 1u) / 3u) big = 0u;
+#pragma unroll
+    for (uint32_t q = 1; q < 4u; ++q) {
+        const bool swap = q == big;
+        const uint32_t s0 = size[0];
+        const int32_t g0 = g[0];
+        size[0] = swap ? size[q] : s0;
+        g[0] = swap ? g[q] : g0;
+        size[q] = swap ? s0 : size[q];
+        g[q] = swap ? g0 : g[q];
+    }
+    float b[4][6];
+    uint32_t ref[4], tag[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool there = size[q] != 0u;
+        const float* src = nullptr;
+        ref[q] = 0xFFFFFFFFu;            // kWideNone
+        tag[q] = 0u;
+        if (there && g[q] >= 0) {
+            const uint32_t item = (uint32_t)keys[g[q]];
+            ref[q] = item | 0x80000000u;        // kWideLeaf
+            tag[q] = __float_as_uint(coll[(size_t)item * 5u + 3u].w) & 0xFFFFu;
+            src = aabbs + (size_t)item * 6u;
+        } else if (there) {
+            ref[q] = (uint32_t)-g[q];
+            src = node_aabb + (size_t)(-g[q]) * 6u;
         }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int q = 2 * h + k;
-            const bool there = k == 0 || two;
-            const float* src = nullptr;
-            ref[q] = 0xFFFFFFFFu;        // kWideNone
-            tag[q] = 0u;
-            if (there && g[k] >= 0) {
-                const uint32_t item = (uint32_t)keys[g[k]];
-                ref[q] = item | 0x80000000u;        // kWideLeaf
-                tag[q] = __float_as_uint(coll[(size_t)item * 5u + 3u].w) & 0xFFFFu;
-                src = aabbs + (size_t)item * 6u;
-            } else if (there) {
-                ref[q] = (uint32_t)-g[k];
-                src = node_aabb + (size_t)(-g[k]) * 6u;
-            }
-#pragma unroll
-            for (int z = 0; z < 6; ++z) b[q][z] = there ? src[z] : (z < 3 ? INFINITY : -INFINITY);
-        }
+        for (int z = 0; z < 6; ++z) b[q][z] = there ? src[z] : (z < 3 ? INFINITY : -INFINITY);
     }
     float4* o = wide + (size_t)i * 8u;
 #pragma unroll
     for (int z = 0; z < 6; ++z) o[z] = make_float4(b[0][z], b[1][z], b[2][z], b[3][z]);
     o[6] = make_float4(__uint_as_float(ref[0]), __uint_as_float(ref[1]), __uint_as_float(ref[2]),
                        __uint_as_float(ref[3]));
-    const uint32_t e = (uint32_t)other_end[i];
-    o[7] = make_float4(__uint_as_float(min(i, e)), __uint_as_float(max(i, e) + 1u),
+    o[7] = make_float4(__uint_as_float(l), __uint_as_float(r + 1u),
                        __uint_as_float(tag[0] | tag[1] << 16), __uint_as_float(tag[2] | tag[3] << 16));
 }
 

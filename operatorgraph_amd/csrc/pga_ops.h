@@ -283,7 +283,12 @@ __device__ __forceinline__ bool collider_test(const float4* __restrict__ coll, u
 // levels (1.2M props against 81,920 colliders: 408 us with 32-byte binary
 // nodes in depth-first order, where every rejected sibling is a load of its
 // own; 293 with these and the lanes' leaves tested together). A node that a
-// full stack could not take the children of is scanned, leaf by leaf.
+// full stack could not take the children of is scanned, leaf by leaf and
+// without a look at their boxes; with the children in the order that k_wide
+// gives them, it holds at most 1/729 of the colliders (or 32). In the tree's
+// own order it could hold nearly all: 16,384 questions over a trail of
+// outliers against a cluster of as many colliders took 14.6 ms (0.52 ms with
+// binary nodes), in this order 0.31 ms.
 __device__ __forceinline__ bool collider_hit(const Ctx& c, uint32_t n, uint32_t tag, uint32_t phase,
                                              uint32_t shape, const float bm[12], const float bs[3],
                                              const CollMemo* memo) {

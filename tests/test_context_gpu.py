@@ -97,6 +97,64 @@ def test_collision_walk_of_overlapping_colliders(E, pairs):
     assert len(got[1]) <= pairs // 2 and len(got[2]) >= (pairs + 1) // 2
 
 
+def _trail(pairs, outliers):
+    """Colliders in a cluster at the scene's high corner, a chain of twins
+    trailing away from it along each axis at doubling distances (`outliers`),
+    all of one tag. The questions are upright sheets that lie across the scene,
+    clear of every collider: their boxes hold all outliers and the cluster's
+    low corner."""
+    rng = np.random.default_rng(5)
+    ax, p = axioms.collision_pair_axioms([(B, B)] * pairs, rng)
+    a, b = p[0::2], p[1::2]
+    a[:, 0:6] = (0.01, 0.01, 0.01, 0.0, 0.0, 0.0)
+    a[:, 6:9] = rng.uniform(0.0, 32.0, (pairs, 3))
+    if outliers:
+        for k in range(30):
+            a[k, 6:9] = 0.0
+            a[k, 6 + k // 2 % 3] = 32.0 - 768.0 / 2 ** (k // 6)
+    reach, w = 1100.0, -1100.0 / 2 + 1.0
+    b[:] = (0.01, reach, 2 ** 0.5 * reach, 0.0, -45.0, 0.0, 2 ** 0.5 * w, w, 0.0, 7.0)
+    a[:, 9] = 7.0
+    return ax, p
+
+
+def test_collision_walk_of_a_trail(E):
+    """A walk whose stack is full of outliers when it comes to the cluster:
+    the same answers as the oracle, questions that do collide among them."""
+    _note("collision walk over a trail")
+    ax, p = _trail(1500, True)
+    rng = np.random.default_rng(6)
+    p[1::4, 0:3] = rng.uniform(0.5, 4.0, (750, 3))
+    p[1::4, 3:6] = rng.uniform(0.0, 360.0, (750, 3))
+    p[1::4, 6:9] = rng.uniform(-30.0, 30.0, (750, 3))
+    got, ref, phases = check(E, grammars.collision_pairs(), ax, 3, params=p)
+    assert phases == 2 and len(got[1]) > 0 and len(got[2]) > 750
+
+
+def test_collision_walk_is_not_a_scan(E):
+    """The trail costs little beside the cluster alone (305 and 265 us for
+    16,384 pairs; 14.6 ms when the walk, its stack full, scanned the cluster
+    leaf by leaf). The bound lies between."""
+    _note("collision walk over a trail, time")
+    best = {}
+    for outliers in (False, True):
+        ax, p = _trail(16384, outliers)
+        eng = E.Engine()
+        try:
+            eng.load(grammars.collision_pairs()).set_axioms(ax).set_axiom_params(p)
+            for t in range(3):
+                eng.bind(t, 16384)
+            times = []
+            for _ in range(6):
+                eng.execute()
+                times.append(eng.kernel_seconds())
+            assert [int(c) for c in eng.counts(3)] == [16384, 0, 16384]
+            best[outliers] = min(times)
+        finally:
+            eng.close()
+    assert best[True] < 5.0 * best[False], best
+
+
 @pytest.mark.parametrize("technique", TECHNIQUES)
 @pytest.mark.parametrize("walls", [False, True])
 def test_context_city(E, technique, walls):
