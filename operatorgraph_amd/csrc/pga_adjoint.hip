@@ -507,7 +507,6 @@ __device__ __forceinline__ Ctx adj_ctx(const KArgs& a, const AdjLDS& T) {
     c.seed = a.use_seed;
     c.poly = 0u;             // the tape refuses dynamic polygons
     c.tape = 1u;
-    c.prog_lds = 1u;
     c.ctxs = 0u;             // one-phase programs without Collider / IfCollides only
     c.dmask = 0xFFFFu;
     c.phase = 0u;
