@@ -79,7 +79,7 @@ def _gpu_run(program, ax, params, n_terms, tape=True):
     return eng
 
 
-def _adjoint_pair(program, ax, params, n_terms):
+def _adjoint_pair(program, ax, params, n_terms, weights=_weights):
     import torch
     from oracle import oracle as O
     eng = _gpu_run(program, ax, params, n_terms)
@@ -87,14 +87,14 @@ def _adjoint_pair(program, ax, params, n_terms):
     dl = {}
     for t in range(n_terms):
         g = np.zeros((len(got[t]), 16), dtype=np.float32)
-        g[:, :12] = _weights(got[t])
+        g[:, :12] = weights(got[t])
         dl[t] = torch.from_numpy(g).cuda()
     grad = eng.backward(dl).cpu().numpy().astype(np.float64)
     r = O.derive(program, ax, params=params, twins=O.TWIN_F64 | O.TWIN_ADJ)
     ref_inst = [r.instances(t) for t in range(n_terms)]
     for t in range(n_terms):
         assert_same_multiset(got[t], ref_inst[t], f"terminal {t}")
-    ref = r.backward([_weights(ref_inst[t]) for t in range(n_terms)])
+    ref = r.backward([weights(ref_inst[t]) for t in range(n_terms)])
     eng.close()
     return grad, ref, r
 
@@ -364,7 +364,9 @@ def test_adjoint_axioms_sharing_a_wave(children):
     """A wave with the children of several axioms sums the parameters axiom by
     axiom, from eight children of one on: Repeat(X, 1) Translate(p0, p1, 0)
     Scale(p2, -1, -1) Generate(0) over `children` tiles each. FP32 terms of
-    both signs: their rounding against the largest parameter of the axiom."""
+    both signs, whose sum can cancel: their rounding is held against the
+    largest parameter of the axiom, and an entry only loosely against itself
+    (the next test holds the sums exactly)."""
     _note(f"adjoint of {children} children an axiom")
     table = DispatchTable([
         Entry(op(abi.REPEAT, Q), [Scalar(abi.X), Scalar(1.0), Scalar(abi.ADJUST_TO_FILL)], [(1, 0)]),
@@ -382,6 +384,43 @@ def test_adjoint_axioms_sharing_a_wave(children):
     grad, ref, r = _adjoint_pair(Program(grammars.INTERPRETER_PROCEDURES, table, "tiles"), ax, params, 1)
     assert r.count(0) == n * children
     _assert_close(grad, ref, rel=1e-4, entry_rel=5e-2)
+
+
+def _whole_weights(inst):
+    """Whole numbers from -2 to 2 by (axiom, path), none of a row's zero."""
+    key = inst["axiom"].astype(np.int64)[:, None] * 31 + (inst["path"].astype(np.int64) % 97)[:, None] * 7
+    w = (key + np.arange(12)[None, :] * 3) % 4 - 2
+    return np.where(w >= 0, w + 1, w).astype(np.float64)
+
+
+@pytest.mark.parametrize("children", [1, 2, 7, 8, 9, 33, 64, 65])
+@pytest.mark.parametrize("slots", [3, 8, 9])
+def test_adjoint_axioms_sharing_a_wave_exactly(children, slots):
+    """The same sums with every term exact: sizes, positions and parameters
+    are multiples of 1/8, weights are whole numbers, so that FP32 terms and
+    FP64 sums have no rounding and the gradients are the oracle's to the last
+    bit. A term lost, doubled or given to another axiom shows. slots: three
+    parameters that are used, at the ends of a row of `slots` (more than eight
+    go past the sums in LDS)."""
+    _note(f"adjoint of {children} children an axiom, {slots} parameters, exactly")
+    last = slots - 1
+    table = DispatchTable([
+        Entry(op(abi.REPEAT, Q), [Scalar(abi.X), Scalar(1.0), Scalar(abi.ADJUST_TO_FILL)], [(1, 0)]),
+        Entry(op(abi.TRANSLATE, Q), [AxiomParam(0), AxiomParam(last), Scalar(0.0)], [(2, 0)]),
+        Entry(op(abi.SCALE, Q), [AxiomParam(1), Scalar(-1.0), Scalar(-1.0)], [(3, 0)]),
+        Entry(op(abi.GENERATE, Q, 1), [Scalar(0)], []),
+    ])
+    n = 37
+    rng = np.random.default_rng(children)
+    ax = axioms.empty(n)
+    ax["size"] = np.stack([np.full(n, float(children)), rng.integers(8, 17, n) / 8.0, np.zeros(n)], axis=1)
+    ax["model"][:, [3, 7, 11]] = rng.integers(-40, 41, size=(n, 3)) / 8.0
+    ax["shape_type"] = Q
+    params = (rng.integers(2, 8, size=(n, slots)) / 8.0).astype(np.float32)
+    grad, ref, r = _adjoint_pair(Program(grammars.INTERPRETER_PROCEDURES, table, "tiles"), ax, params, 1,
+                                 weights=_whole_weights)
+    assert r.count(0) == n * children and np.abs(ref).max() > 0
+    assert np.array_equal(grad, ref), np.abs(grad - ref).max()
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 511, 513, 512 * 512 - 1, 512 * 512 + 65])

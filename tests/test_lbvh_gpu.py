@@ -77,6 +77,54 @@ def test_lbvh_tile_edges(n, boxes):
     _compare(_gpu_build(b, smin, smax), O.lbvh(b, smin, smax), n)
 
 
+@pytest.mark.parametrize("bound,n", [(4096, n) for n in (1, 2, 1023, 1024, 1025, 4095, 4096)] +
+                         [(65537, n) for n in (1, 2, 1023, 1024, 1025, 4095, 4096, 4097, 8193, 32769, 65537)])
+def test_lbvh_device_count_edges(bound, n):
+    """The leaf count on the device, under a bound that launches more
+    workgroups than there are tiles: empty sort tiles, empty groups of the
+    tree, and the one-workgroup sort. What lies past the count stays as it
+    was."""
+    import torch
+    from operatorgraph_amd import abi, engine
+    from operatorgraph_amd.lbvh import LBVH
+    from operatorgraph_amd.program import DispatchTable, Entry, Program, Scalar
+    _note(f"lbvh device count n={n} bound={bound}")
+    rng = np.random.default_rng(n)
+    ax = axioms.empty(n)
+    ax["size"] = rng.uniform(0.1, 2.0, size=(n, 3)).astype(f32)
+    ax["model"][:, [3, 7, 11]] = rng.uniform(-50, 50, size=(n, 3)).astype(f32)
+    ax["shape_type"] = abi.BOX
+    table = DispatchTable([Entry(grammars.op(abi.GENERATE, abi.BOX, 1), [Scalar(0)], [])])
+    eng = engine.Engine()
+    eng.load(Program(grammars.INTERPRETER_PROCEDURES, table, "boxes")).set_axioms(ax)
+    eng.bind(0, n)
+    eng.execute()
+    b = LBVH(bound, engine=eng)
+    out = b.alloc()
+    for v in out.values():
+        v.fill_(-77)
+    torch.cuda.synchronize()
+    b.gather_engine(eng, 1, 0, out)
+    b.build_device(out)
+    assert b.leaf_count() == (n, False)
+    got = {k: v.cpu().numpy() for k, v in out.items()}
+    boxes = got["aabbs"][:n]
+    inst = eng.instances(0)
+    assert np.array_equal(boxes.view(np.uint32), _np_instance_boxes(inst, False).view(np.uint32))
+    smin, smax = boxes[:, :3].min(0), boxes[:, 3:].max(0)
+    if n > 1:
+        ref = O.lbvh(boxes, smin, smax)
+        cut = {k: got[k][: n if k in ("keys", "leaf_parent") else n - 1] for k in ref}
+        _compare(cut, ref, n)
+    else:
+        assert got["keys"][0] & 0xFFFFFFFF == 0
+    for k in ("keys", "leaf_parent", "left", "right", "parent", "node_aabb"):
+        rest = got[k][n if k in ("keys", "leaf_parent") else n - 1 :]
+        assert np.all(rest == -77), k
+    b.close()
+    eng.close()
+
+
 def _np_instance_boxes(inst, planar):
     m = inst["model"].astype(f32)
     h = [np.abs(m[:, 4 * r]) + np.abs(m[:, 4 * r + 1]) for r in range(3)]

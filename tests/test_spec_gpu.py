@@ -111,6 +111,89 @@ def test_spec_leaf_fans(children):
         assert [len(g) for g in got] == [n * succ.count(WALL), n * succ.count(WINDOW)]
 
 
+def _direct_program(pad):
+    """Direct leaf fan-outs of every kind, as separate entry points 0 to 4:
+    a Subdivide over terminals 0 and 1 (every fifth child dropped), one over 2
+    and 3, a Repeat of terminal 1, a ComponentSplit of one terminal for caps
+    and another for sides, and one that drops the top. pad: more Subdivides,
+    for a program whose entries are grouped."""
+    from operatorgraph_amd.program import DispatchTable, Entry, Program, Scalar
+    Q = abi.QUAD
+    BOX0, QUAD4, NONE_B, NONE_Q = 5, 9, 11, 12
+    entries = [
+        grammars.subdiv_entry(B, abi.X, [-1.0, -2.0, 0.1, -0.5, -1.5], [BOX0, BOX0 + 1, BOX0, BOX0 + 1, NONE_B]),
+        grammars.subdiv_entry(B, abi.Y, [-1.0, -1.0, -3.0], [BOX0 + 3, BOX0 + 2, BOX0 + 3]),
+        Entry(grammars.op(abi.REPEAT, B), [Scalar(abi.Z), Scalar(0.17), Scalar(abi.ADJUST_TO_FILL)], [(BOX0 + 1, 0)]),
+        Entry(grammars.op(abi.COMPSPLIT, B), [], [(QUAD4, 0), (QUAD4, 0), (QUAD4 + 1, 0)]),
+        Entry(grammars.op(abi.COMPSPLIT, B), [], [(NONE_Q, 0), (QUAD4 + 1, 0), (QUAD4, 0)]),
+    ]
+    entries += [Entry(grammars.op(abi.GENERATE, B, 1), [Scalar(t)], []) for t in range(4)]
+    entries += [Entry(grammars.op(abi.GENERATE, Q, 1), [Scalar(t)], []) for t in (4, 5)]
+    entries += [Entry(grammars.op(abi.DISCARD, B), [], []), Entry(grammars.op(abi.DISCARD, Q), [], [])]
+    points = list(range(5))
+    for k in range(pad):
+        points.append(len(entries))
+        entries.append(grammars.subdiv_entry(B, k % 3, [-1.0, -1.0 - 0.25 * k, -0.5],
+                                             [BOX0 + k % 4, BOX0 + (k + 1 + k // 4) % 4, BOX0 + k % 4]))
+    return Program(grammars.INTERPRETER_PROCEDURES, DispatchTable(entries), f"direct{pad}"), points
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 300])
+@pytest.mark.parametrize("only", [2, 3, 4, None])
+@pytest.mark.parametrize("pad", [0, 24])
+def test_spec_direct_fans(n, only, pad):
+    """Direct leaf fan-outs, alone (a Repeat's rounds are counted at run time,
+    a ComponentSplit's children take its successors in an order of their own)
+    and all mixed in every wave."""
+    _note(f"specialised: direct fan-outs n={n} only={only} pad={pad}")
+    prog, points = _direct_program(pad)
+    assert (len(prog.table.entries) > 32) == (pad > 0)      # more than 32 entries: types are grouped
+    ax = _boxes(n, 31 + n)
+    ax["entry_index"] = [points[i % len(points)] if only is None else only for i in range(n)]
+    spec_check(prog, ax, 6)
+
+
+@pytest.mark.parametrize("short", [0, 1])
+@pytest.mark.parametrize("room", [0, 1, 5, 64, 100])
+def test_spec_direct_fan_overflows_one_terminal(short, room):
+    """A direct fan-out of two terminals with one buffer too small: the status
+    says so, both counts are whole, the other terminal's records are all
+    there and so are those that fit, and nothing is written past them."""
+    import torch
+    from oracle import oracle as O
+    from operatorgraph_amd import engine
+    from tests.helpers import canon
+    _note(f"specialised: overflow of terminal {short} at {room}")
+    prog, points = _direct_program(0)
+    n = 130
+    ax = _boxes(n, 37)
+    ax["entry_index"] = points[0]
+    r = O.derive(prog, ax)
+    eng = engine.Engine()
+    try:
+        eng.load(prog).set_axioms(ax)
+        other = 1 - short
+        eng.bind(other, r.count(other))
+        guard = torch.full((room + 64, 16), 7.0, device="cuda")
+        eng.bind(short, room, guard if room else None)
+        eng.specialize()
+        if room:
+            with pytest.raises(engine.PGAError) as e:
+                eng.execute()
+            assert e.value.status == abi.ERR_OVERFLOW_INSTANCES
+        else:
+            eng.execute()                        # capacity 0 counts only
+        assert [int(c) for c in eng.counts(2)] == [r.count(0), r.count(1)]
+        assert_same_multiset(eng.instances(other), r.instances(other), "the terminal with room")
+        if room:
+            rows = {row.tobytes() for row in canon(r.instances(short))}
+            kept = canon(eng.instances(short, room))
+            assert len(kept) == room and all(row.tobytes() in rows for row in kept)
+            assert bool((guard[room:] == 7.0).all())
+    finally:
+        eng.close()
+
+
 @pytest.mark.parametrize("name", sorted(k for k, v in grammar_fixture().items() if "refused" not in v))
 def test_spec_reference_grammar(name):
     _note(f"specialised: reference grammar {name}")
