@@ -174,7 +174,10 @@ struct pga_graph {
 namespace {
 
 const uint32_t kDefaultCapacity = 1u << 22;
-const uint32_t kDefaultColliders = 1u << 20;   // 80 MB of collider store
+// 84 MB of collider store and, for more than one phase, about 230 MB for the
+// tree over it: per collider 24 B of box, 8 of key, 40 of binary tree, 128 of
+// four-wide node and 20 of build scratch
+const uint32_t kDefaultColliders = 1u << 20;
 const uint32_t kDefaultMaxLevels = 4096;
 const uint32_t kMaxChain = 256;
 const uint32_t kMaxProgramLds = 60u * 1024u;   // program image + terminal tables

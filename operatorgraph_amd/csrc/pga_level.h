@@ -77,20 +77,6 @@ __device__ __forceinline__ uint32_t claim(LevelLDS& L, bool wr, uint32_t k, unsi
     return base;
 }
 
-// GenerationFunction<GenFuncFilter, 1>::perShape (GenerationFunctions.cuh:
-// 155-189): instance = model4 * scale(size), custom attribute. A full buffer
-// is an error (the reference wraps modulo capacity); capacity 0 counts only.
-// The lanes of one claim get consecutive records, so the write pass stages
-// them in the wave's part of LDS (ST, 64 records) in rank order and writes
-// them out as consecutive 16-byte nontemporal stores: a lane storing its own
-// record would leave every store instruction a 64-byte stride, and partly
-// written lines cost more than the coalesced stream (measured 0.91 -> 0.80 ms
-// on 16,384 facade lots). The four words of record r are rotated by r / 4
-// (stage_at), so that 16 lanes of either side of the copy touch 16 different
-// 16-byte columns of LDS: in place, the lanes writing word k of 16 records
-// met on four of them (41M conflict cycles on 16,384 lots). The copy reads its (at most four) words per lane
-// from LDS before any store, and stores through a global-memory pointer: a
-// flat store would also count against the LDS wait of the next read.
 // The instance record of a terminal shape as four 16-byte rows: model4 *
 // scale(size) (rows 0-2), then custom attribute, axiom, path and entry |
 // depth << 16.
@@ -122,7 +108,18 @@ __device__ __forceinline__ void instance_rows(const Rec& r, bool inv, f4& q0, f4
 __device__ __forceinline__ uint32_t stage_at(uint32_t r, uint32_t k) { return r * 4u + ((k + (r >> 2)) & 3u); }
 
 // Stages the records of the lanes in `mask` (rank: the lane's among them) and
-// writes them out from dst on; records at or past `room` stay out.
+// writes them out from dst on; records at or past `room` stay out. The lanes of
+// one claim get consecutive records, so they are staged in the wave's part of
+// LDS (ST, 64 records) in rank order and written out as consecutive 16-byte
+// nontemporal stores: a lane storing its own record would leave every store
+// instruction a 64-byte stride, and partly written lines cost more than the
+// coalesced stream (measured 0.91 -> 0.80 ms on 16,384 facade lots). The four
+// words of record r are rotated by r / 4 (stage_at), so that 16 lanes of either
+// side of the copy touch 16 different 16-byte columns of LDS: in place, the
+// lanes writing word k of 16 records met on four of them. The copy reads its
+// (at most four) words per lane from LDS before any store, and stores through a
+// global-memory pointer: a flat store would also count against the LDS wait of
+// the next read.
 __device__ __forceinline__ void copy_out(f4* ST, gf4* dst, unsigned long long room, bool mine, uint32_t rank,
                                          unsigned long long mask, f4 q0, f4 q1, f4 q2, f4 q3) {
     if (mine) {
@@ -151,6 +148,9 @@ __device__ __forceinline__ void copy_out(f4* ST, gf4* dst, unsigned long long ro
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// GenerationFunction<GenFuncFilter, 1>::perShape (GenerationFunctions.cuh:
+// 155-189): instance = model4 * scale(size), custom attribute. A full buffer
+// is an error (the reference wraps modulo capacity); capacity 0 counts only.
 __device__ __forceinline__ void emit_terminal(const Ctx& c, LevelLDS& L, f4* ST, bool wr, bool has, uint32_t slot,
                                               const Rec& r, unsigned long long& idx) {
     f4 q0 = {}, q1 = {}, q2 = {}, q3 = {};

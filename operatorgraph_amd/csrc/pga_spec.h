@@ -519,6 +519,12 @@ __device__ __forceinline__ void spec_mega(const KArgs& a) {
             nwaves = blockDim.x >> 6;
         } else {
             io = grid_io(a, level);
+            // consecutive waves in a block: a level's neighbours share parents, and
+            // a wide level reads them once per block (16,384 lots, grid-wide at 768
+            // threads: 470 us, 488 with the interpreting kernels' order, which
+            // gains where a level is narrow: 1,024 lots 128 and 119, the
+            // stochastic batch 443 and 419). The workgroups' own levels leave
+            // the wide ones to this path.
             wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
             nwaves = (gridDim.x * blockDim.x) >> 6;
         }
