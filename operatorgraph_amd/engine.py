@@ -203,7 +203,8 @@ class Engine:
         torch = self.torch
         if isinstance(params, torch.Tensor) and params.is_cuda and \
                 params.device.index == torch.cuda.current_device() == self._device:
-            p = params.detach().to(torch.float32).contiguous()
+            # a negative or conjugate view holds other bits than its values
+            p = params.detach().resolve_conj().resolve_neg().to(torch.float32).contiguous()
             self._after_torch()
             self._check(self.L.pga_set_axiom_params(self._h, C.c_void_p(p.data_ptr()), p.shape[0], p.shape[1]))
             self.params_per_axiom = p.shape[1]

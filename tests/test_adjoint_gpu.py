@@ -468,3 +468,30 @@ def test_axiom_params_from_device_tensors():
         for t in range(2):
             assert_same_multiset(eng.instances(t), want[t], f"terminal {t}")
     eng.close()
+
+
+@pytest.mark.parametrize("form", ["negative", "imaginary"])
+def test_axiom_params_from_lazy_views(form):
+    """Device tensors whose memory does not hold their values (torch's negative
+    views, the imaginary part of a conjugate) bind their values, too."""
+    import torch
+    from operatorgraph_amd import engine
+    _note(f"axiom parameters from a {form} view")
+    ax, params = axioms.param_lots(24, perturb=0.05)
+    dev = torch.from_numpy(params).cuda()
+    if form == "negative":
+        view = torch._neg_view(-dev)
+    else:
+        view = torch.complex(torch.zeros_like(dev), -dev).conj().imag
+    assert view.is_neg() and torch.equal(view, dev)
+    eng = engine.Engine(queue_capacity=1 << 20)
+    eng.load(grammars.facade_params()).set_axioms(ax).set_axiom_params(view)
+    for t in range(2):
+        eng.bind(t, 1 << 18)
+    eng.execute()
+    got = [eng.instances(t) for t in range(2)]
+    eng.set_axiom_params(params)
+    eng.execute()
+    for t in range(2):
+        assert_same_multiset(got[t], eng.instances(t), f"terminal {t}")
+    eng.close()
