@@ -568,7 +568,8 @@ __device__ __forceinline__ void child_start(const KArgs& a, const AdjArgs& g, co
 // one record at a time and derives it again from the tape where it needs it
 // later (the parent is in L2), instead of the parent, the starting state and
 // the end of the chain side by side. Slots are 64 bytes and leave through LDS:
-// stored lane by lane, 312 MB of them became 716 MB of writes. The levels of
+// stored lane by lane, the 312 MB of the last level's became 716 MB of writes
+// (502 MB now, scratch included). The levels of
 // 4,096 parameterised lots, last first: 372 / 661 / 295 / 67 us with 80-byte
 // slots, the program read from memory and 48 bytes of scratch a lane; 299 /
 // 559 / 227 / 52 us with that; 297 / 434 / 190 / 60 with the gradient sums in
