@@ -110,7 +110,8 @@ struct pga_context {
     uint32_t* d_coll_count = nullptr;
     uint32_t colliders = 0;           // stored by the last execute
     // LBVH over the colliders, built between phases (multi-phase programs):
-    // leaf boxes, keys, children, parents and node boxes for coll_cap leaves
+    // leaf boxes, keys, children, parents and node boxes for coll_cap leaves;
+    // there only if coll_bvh_cap == coll_cap
     pga_lbvh* coll_bvh = nullptr;
     uint32_t coll_bvh_cap = 0;
     float* d_coll_boxes = nullptr;
@@ -810,6 +811,9 @@ pga_status ensure_colliders(pga_context* ctx) {
         if (ctx->stream) HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
         hfree(ctx->d_coll);
         ctx->coll_cap = 0;
+        // the tree goes with its store, whose colliders its nodes are made from:
+        // built for another bound, it would read past a smaller store's end
+        drop_collider_bvh(ctx);
         HIP_TRY(ctx, hipMalloc((void**)&ctx->d_coll, (size_t)want * 5u * sizeof(float4)));
         ctx->coll_cap = want;
     }

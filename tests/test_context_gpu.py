@@ -215,6 +215,43 @@ def test_collider_capacity_overflow(E):
         eng.close()
 
 
+@pytest.mark.parametrize("technique", TECHNIQUES)
+@pytest.mark.parametrize("capacity", [1, 2, 32, 33, 2000])
+def test_collider_capacity_lowered(E, technique, capacity):
+    """A store made smaller than the one before, down to a single collider
+    (for which no tree is built), with more colliders than it holds, then as
+    many as it holds, and the default again."""
+    from oracle import oracle as O
+    _note(f"collider capacity lowered to {capacity}, technique={technique}")
+    lots = axioms.city_lots(3000)
+    prog = grammars.context_city()
+    few = lots[:min(capacity, 48)]
+    ref_few = O.derive(prog, few)
+    eng = E.Engine(technique=technique)
+    try:
+        eng.load(prog).set_axioms(lots)
+        for t in range(3):
+            eng.bind(t, 1 << 18)
+        eng.execute()
+        counts = [int(c) for c in eng.counts(3)]
+        assert eng.colliders()[0] == len(lots)
+        eng.set_collider_capacity(capacity)
+        with pytest.raises(E.PGAError) as e:
+            eng.execute()
+        assert e.value.status == abi.ERR_OVERFLOW_QUEUE
+        eng.set_axioms(few)
+        eng.execute()
+        for t in range(3):
+            assert_same_multiset(eng.instances(t), ref_few.instances(t), f"terminal {t}")
+        assert eng.colliders()[0] == len(few)
+        eng.set_collider_capacity(0)
+        eng.set_axioms(lots)
+        eng.execute()
+        assert [int(c) for c in eng.counts(3)] == counts
+    finally:
+        eng.close()
+
+
 def test_refusals(E):
     _note("context-sensitive programs: specialise, tape and capture refused; phase 16 rejected")
     eng = E.Engine()
